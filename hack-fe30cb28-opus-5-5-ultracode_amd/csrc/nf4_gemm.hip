@@ -7,13 +7,14 @@
 //   NN (backward): C[m, n] = sum_k A[m, k] B[k, n]      B = W [K, N], N = W's columns
 //
 // One workgroup = 4 wavefronts on a 256 x 256 output tile; each wavefront owns a 128 x 128
-// block as 4 x 4 v_mfma_f32_32x32x16_f16 accumulators (256 accumulation registers, one
-// wavefront per SIMD). Two main loops share the tile, the MFMA order and the epilogues: the NF4
-// one (nf4_gemm_kernel, k-tiles of 32, four LDS stages, described below) and the fp16-B one
-// (hgemm_kernel, k-tiles of 64, two stages: every DMA lane group then fetches whole 128-byte
-// lines, which the L1 serves at twice the rate of 64-byte halves; described at the kernel). On gfx950 a 128 x 128 wavefront block is what keeps the operand reads
+// block (256 accumulation registers, one wavefront per SIMD). Two main loops share the tile, the
+// order of each output's sum and the epilogues: the NF4 one (nf4_gemm_kernel, 4 x 4
+// v_mfma_f32_32x32x16_f16 a k-step, k-tiles of 32, four LDS stages, described below) and the
+// fp16-B one (hgemm256_kernel, 8 x 8 v_mfma_f32_16x16x32_f16, k-tiles of 64: every DMA lane group
+// then fetches whole 128-byte lines, which the L1 serves at twice the rate of 64-byte halves;
+// described at the kernel). On gfx950 a 128 x 128 wavefront block is what keeps the operand reads
 // below the MFMA time: per 16-wide k-step a wavefront reads 2 x 128 x 16 fp16 from LDS for 16
-// MFMAs; smaller blocks make the kernel LDS-bound.
+// MFMAs of 32 x 32; smaller blocks make the kernel LDS-bound.
 //
 // Operand staging (NF4 kernel). The A tile goes from global memory straight into LDS
 // (global_load_lds_dwordx4: a wavefront instruction writes 1 KB of consecutive LDS, lane l at
@@ -66,6 +67,7 @@ namespace qlora {
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) short4_t lds_short4_t;
 typedef __attribute__((address_space(3))) void lds_void_t;
@@ -123,6 +125,7 @@ struct GemmArgs {
   int64_t ldgu;
   float alpha;              // kEpiF32: scale of the product
   const float* row_scale;   // kEpiF32: fp32 [M] scale of each resid row, or null (1)
+  int wide;                 // kEpiF32: c's (and resid's) rows in whole 16-byte pieces
 };
 
 // ---- swizzled LDS offsets (in halves) ---------------------------------------------------------
@@ -140,18 +143,40 @@ __device__ __forceinline__ int tile_order(int b, int total) {
   return b < full ? (b % 8) * (full / 8) + b / 8 : b;
 }
 
+// Tile t of one K slice -> (M tile, N tile): M tiles in groups of at most 12 (the groups as even
+// as they go), a group's M tiles fastest, then the N tiles. An XCD works on 32 consecutive tiles
+// at a time, and what its L2 must bring in per k-tile is their M tiles plus their N tiles: with
+// all 16 M tiles of 4,001 rows fastest it is 16 + 2 operand blocks of 32 KB, in two groups of 8
+// it is 8 + 4 (the [4001, 3584] x [37888, 3584] SwiGLU product 1,039 -> 1,011 us). Up to 12 M
+// tiles (3,072 rows) one group is as good and reads B once.
+__device__ __forceinline__ void tile_pos_lane(int t, int m_tiles, int n_tiles, int& tm, int& tn) {
+  const int groups = (m_tiles + 11) / 12, gm = (m_tiles + groups - 1) / groups;
+  const int grp = t / (gm * n_tiles);
+  t -= grp * gm * n_tiles;
+  const int w = min(gm, m_tiles - grp * gm);
+  tm = grp * gm + t % w;
+  tn = t / w;
+}
+// The same for a wave-uniform t, in scalar registers.
+__device__ __forceinline__ void tile_pos(int t, int m_tiles, int n_tiles, int& tm, int& tn) {
+  tile_pos_lane(t, m_tiles, n_tiles, tm, tn);
+  tm = __builtin_amdgcn_readfirstlane(tm);
+  tn = __builtin_amdgcn_readfirstlane(tn);
+}
+
 // The workgroup's (M tile, N tile, K slice), in scalar registers: the values are the same for
 // every lane, and held in VGPRs across the main loop they cost registers the loop needs. The
-// grid is one-dimensional, the K slices included (slice-major, then N tile, then M tile), so
+// grid is one-dimensional, the K slices included (slice-major, then tile_pos's order), so
 // the XCD order above gives each XCD a run of tiles of one K slice: its L2 then holds the few
 // A and B blocks of that K range which its workgroups share.
 __device__ __forceinline__ void tile_of(int m_tiles, int tiles, int total, int64_t& tile_m,
                                         int64_t& tile_n, int& slice) {
   int t = tile_order(blockIdx.x, total);  // the grid is below 2^31 (host check)
   slice = __builtin_amdgcn_readfirstlane(t / tiles);
-  t -= slice * tiles;
-  tile_m = __builtin_amdgcn_readfirstlane(t % m_tiles);
-  tile_n = __builtin_amdgcn_readfirstlane(t / m_tiles);
+  int tm, tn;
+  tile_pos(t - slice * tiles, m_tiles, tiles / m_tiles, tm, tn);
+  tile_m = tm;
+  tile_n = tn;
 }
 
 // ---- global -> LDS (DMA) ----------------------------------------------------------------------
@@ -288,6 +313,33 @@ struct FragsT {
 };
 typedef FragsT<4, 4> Frags;
 
+// The accumulators of a wavefront's block as groups of four consecutive columns of a row, a lane's
+// in row block i: group g (0 .. CG - 1) is row row(i), columns col(g) .. + 3 of the block, values
+// get(i, g, 0 .. 3). Both forms hold transposed products (B's fragment as the MFMA's first
+// operand), which is what makes the four columns one lane's. SwiGLU: group g's up columns are
+// group g + CG / 2.
+// FM x FN MFMA blocks of 32 x 32 (mfma_step).
+template <int FM, int FN>
+struct Acc32 {
+  static constexpr int RB = FM, CG = 4 * FN;
+  f32x16 a[FM][FN];
+  static __device__ __forceinline__ int row(int i, int lane) { return 32 * i + (lane & 31); }
+  static __device__ __forceinline__ int col(int g, int lane) {
+    return 32 * (g >> 2) + 8 * (g & 3) + 4 * (lane >> 5);
+  }
+  __device__ __forceinline__ float get(int i, int g, int e) const {
+    return a[i][g >> 2][4 * (g & 3) + e];
+  }
+};
+// 8 x 8 MFMA blocks of 16 x 16 (a 128 x 128 block).
+struct Acc16 {
+  static constexpr int RB = 8, CG = 8;
+  f32x4 a[8][8];
+  static __device__ __forceinline__ int row(int i, int lane) { return 16 * i + (lane & 15); }
+  static __device__ __forceinline__ int col(int g, int lane) { return 16 * g + 4 * (lane >> 4); }
+  __device__ __forceinline__ float get(int i, int g, int e) const { return a[i][g][e]; }
+};
+
 template <bool NN>
 __device__ __forceinline__ void read_frags(Frags& f, const uint16_t* sa, const uint16_t* sb,
                                            int s, int wm, int wn, int lane) {
@@ -316,18 +368,17 @@ __device__ __forceinline__ void read_frags(Frags& f, const uint16_t* sa, const u
   }
 }
 
-// T: the accumulators hold the transposed blocks (B fragments as the MFMA's first operand), so
-// register r of lane l in block (i, j) is row 32 i + l % 32, column 32 j + 8 (r / 4) + 4 (l / 32)
-// + r % 4: four consecutive output columns per lane, stored as one 8-byte LDS write. Otherwise
-// register r is row 32 i + 8 (r / 4) + 4 (l / 32) + r % 4, column 32 j + l % 32.
-template <bool T, int FM, int FN>
-__device__ __forceinline__ void mfma_step(f32x16 (&acc)[FM][FN], const FragsT<FM, FN>& f) {
+// The accumulators hold the transposed blocks (B fragments as the MFMA's first operand): register
+// r of lane l in block (i, j) is row 32 i + l % 32, column 32 j + 8 (r / 4) + 4 (l / 32) + r % 4,
+// four consecutive output columns per lane.
+template <int FM, int FN>
+__device__ __forceinline__ void mfma_step(Acc32<FM, FN>& acc, const FragsT<FM, FN>& f) {
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j)
-      acc[i][j] = T ? __builtin_amdgcn_mfma_f32_32x32x16_f16(f.b[j], f.a[i], acc[i][j], 0, 0, 0)
-                    : __builtin_amdgcn_mfma_f32_32x32x16_f16(f.a[i], f.b[j], acc[i][j], 0, 0, 0);
+      acc.a[i][j] =
+          __builtin_amdgcn_mfma_f32_32x32x16_f16(f.b[j], f.a[i], acc.a[i][j], 0, 0, 0);
 }
 
 // Scheduling of one k-step: the reads of the next k-step's fragments between this k-step's 16
@@ -386,32 +437,29 @@ __device__ __forceinline__ void sync_tile() {
 // the same accumulators is formed, one group of four values a lane per 16-byte store, and kept
 // packed in registers; then m is staged in the same LDS area and stored. The values are those of
 // epilogue 3 and of a plain store of the product, bit for bit.
-template <int BM, int BN>
-__device__ __forceinline__ void store_swiglu_keep(const GemmArgs& g,
-                                                  f32x16 (&acc)[BM / 64][BN / 64], uint16_t* lo,
+template <int BM, int BN, typename Acc>
+__device__ __forceinline__ void store_swiglu_keep(const GemmArgs& g, const Acc& acc, uint16_t* lo,
                                                   uint16_t* hi, int64_t m0, int64_t tile_n,
                                                   int lane, int wave) {
-  constexpr int FM = BM / 64, FN = BN / 64, WR = BM / 2, WC = BN / 2, kHalf = WR / 2;
+  constexpr int RB = Acc::RB, CG = Acc::CG, WR = BM / 2, WC = BN / 2, kHalf = WR / 2;
   constexpr int kCh2 = WC / 8, kRows2 = 64 / kCh2, kIt = WR / kRows2;
-  constexpr int kGroups = FM * 4 * (FN / 2), kPer = kGroups / kIt;
+  constexpr int kGroups = RB * (CG / 2), kPer = kGroups / kIt;
   static_assert(kGroups % kIt == 0, "whole groups of SwiGLU values per store");
-  const int wm = wave >> 1, wn = wave & 1, col_in = lane & 31, c4 = 4 * (lane >> 5);
+  const int wm = wave >> 1, wn = wave & 1;
   auto stage2 = [&](int row, int chunk) {
     return (row % kHalf) * WC + ((chunk ^ (row & (kCh2 - 1))) << 3);
   };
 #pragma unroll
-  for (int i = 0; i < FM; ++i) {
-    const int row = i * 32 + col_in;
-    uint16_t* base = i < FM / 2 ? lo : hi;
+  for (int i = 0; i < RB; ++i) {
+    const int row = Acc::row(i, lane);
+    uint16_t* base = i < RB / 2 ? lo : hi;
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        const int col = j * 32 + 8 * q + c4;
-        *reinterpret_cast<uint2*>(base + stage2(row, col >> 3) + c4) =
-            make_uint2(pack2h(acc[i][j][4 * q], acc[i][j][4 * q + 1]),
-                       pack2h(acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]));
-      }
+    for (int q = 0; q < CG; ++q) {
+      const int col = Acc::col(q, lane);
+      *reinterpret_cast<uint2*>(base + stage2(row, col >> 3) + (col & 7)) =
+          make_uint2(pack2h(acc.get(i, q, 0), acc.get(i, q, 1)),
+                     pack2h(acc.get(i, q, 2), acc.get(i, q, 3)));
+    }
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the wavefront's own LDS stores
   const int64_t g_base = tile_n * (BN / 2) + wn * (WC / 2);
@@ -419,7 +467,7 @@ __device__ __forceinline__ void store_swiglu_keep(const GemmArgs& g,
     const int row = k * kRows2 + lane / kCh2, chunk = lane % kCh2;
     return *reinterpret_cast<const uint4*>((row < kHalf ? lo : hi) + stage2(row, chunk));
   };
-  uint2 mv[kGroups];  // group (i, q, j): four m values of row 32 i + l % 32, packed
+  uint2 mv[kGroups];  // group gi: the four m values of row block gi / (CG / 2), packed
   uint4 v = gu_piece(0);
 #pragma unroll
   for (int k = 0; k < kIt; ++k) {
@@ -427,13 +475,12 @@ __device__ __forceinline__ void store_swiglu_keep(const GemmArgs& g,
     if (k + 1 < kIt) vn = gu_piece(k + 1);
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
-      const int gi = k * kPer + u, i = gi / (4 * (FN / 2)), q = (gi / (FN / 2)) % 4,
-                j = gi % (FN / 2);
+      const int gi = k * kPer + u, i = gi / (CG / 2), q = gi % (CG / 2);
       float m[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float gt = h2f(f2h(acc[i][j][4 * q + e]));
-        const float up = h2f(f2h(acc[i][j + FN / 2][4 * q + e]));
+        const float gt = h2f(f2h(acc.get(i, q, e)));
+        const float up = h2f(f2h(acc.get(i, q + CG / 2, e)));
         m[e] = gt * sigmoid_fast(gt) * up;  // as glu_fwd_kernel
       }
       mv[gi] = make_uint2(pack2h(m[0], m[1]), pack2h(m[2], m[3]));
@@ -457,9 +504,9 @@ __device__ __forceinline__ void store_swiglu_keep(const GemmArgs& g,
   __builtin_amdgcn_s_waitcnt(0xC07F);
 #pragma unroll
   for (int gi = 0; gi < kGroups; ++gi) {
-    const int i = gi / (4 * (FN / 2)), q = (gi / (FN / 2)) % 4, j = gi % (FN / 2);
-    const int row = i * 32 + col_in, col = j * 32 + 8 * q + c4;
-    *reinterpret_cast<uint2*>((i < FM / 2 ? lo : hi) + stage_off(row, col >> 3) + c4) = mv[gi];
+    const int i = gi / (CG / 2), row = Acc::row(i, lane), col = Acc::col(gi % (CG / 2), lane);
+    *reinterpret_cast<uint2*>((i < RB / 2 ? lo : hi) + stage_off(row, col >> 3) + (col & 7)) =
+        mv[gi];
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);
   const int64_t n_base = tile_n * (BN / 2) + wn * (WC / 2);
@@ -474,22 +521,20 @@ __device__ __forceinline__ void store_swiglu_keep(const GemmArgs& g,
   }
 }
 
-// The epilogue of a BM x BN tile from the accumulators of mfma_step (4 wavefronts, each on a
-// WR x WC block, WR = BM / 2, WC = BN / 2; register layouts as mfma_step): fp16 outputs are
+// The epilogue of a BM x BN tile from its accumulators (4 wavefronts, each on a
+// WR x WC block, WR = BM / 2, WC = BN / 2; Acc: its accumulators): fp16 outputs are
 // staged through LDS (`lo`: the wavefront's rows 0 .. WR/2 - 1, `hi`: the rest, [WR/2][columns]
 // each, free for this wavefront's use) and leave as whole 16-byte row pieces (the fp32 residual
 // output as 32-byte pieces); split-K partials are stored from the registers.
-template <int EPI, int BM = kBM, int BN = kBN>
-__device__ __forceinline__ void store_tile(const GemmArgs& g, f32x16 (&acc)[BM / 64][BN / 64],
-                                           uint16_t* lo, uint16_t* hi, int64_t m0,
-                                           int64_t tile_n, int lane, int wave, int slice = 0) {
-  constexpr int FM = BM / 64, FN = BN / 64, WR = BM / 2, WC = BN / 2;
-  constexpr bool kT = staged_epi(EPI);
+template <int EPI, int BM = kBM, int BN = kBN, typename Acc>
+__device__ __forceinline__ void store_tile(const GemmArgs& g, const Acc& acc, uint16_t* lo,
+                                           uint16_t* hi, int64_t m0, int64_t tile_n, int lane,
+                                           int wave, int slice = 0) {
+  constexpr int RB = Acc::RB, CG = Acc::CG, WR = BM / 2, WC = BN / 2;
   const int wm = wave >> 1, wn = wave & 1;
-  const int col_in = lane & 31;
   if constexpr (EPI == kEpiSwigluKeep) {
     store_swiglu_keep<BM, BN>(g, acc, lo, hi, m0, tile_n, lane, wave);
-  } else if constexpr (kT) {
+  } else if constexpr (staged_epi(EPI)) {
     // each wavefront writes its block to LDS as fp16 (8-byte LDS stores of four columns,
     // 16-byte chunks XOR-swizzled by row so the 32 rows of a store spread over the banks), then
     // stores whole rows to memory with 16-byte stores
@@ -499,44 +544,27 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, f32x16 (&acc)[BM /
     auto stage_off = [&](int row, int chunk) {
       return (row % kHalf) * kCols + ((chunk ^ (row & (kChunks - 1))) << 3);
     };
-    const int c4 = 4 * (lane >> 5);  // first of the lane's four columns in an 8-column group
 #pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      const int row = i * 32 + col_in;
-      uint16_t* base = i < FM / 2 ? lo : hi;
+    for (int i = 0; i < RB; ++i) {
+      const int row = Acc::row(i, lane);
+      uint16_t* base = i < RB / 2 ? lo : hi;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {  // 8-column group q of each 32-column block
-        if constexpr (swiglu_epi(EPI)) {
+      for (int q = 0; q < (swiglu_epi(EPI) ? CG / 2 : CG); ++q) {
+        const int col = Acc::col(q, lane);
+        float v[4];
 #pragma unroll
-          for (int j = 0; j < FN / 2; ++j) {
-            const int col = j * 32 + 8 * q + c4;
-            float m[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float gt = h2f(f2h(acc[i][j][4 * q + e]));
-              const float up = h2f(f2h(acc[i][j + FN / 2][4 * q + e]));
-              m[e] = gt * sigmoid_fast(gt) * up;  // as glu_fwd_kernel
-            }
-            *reinterpret_cast<uint2*>(base + stage_off(row, col >> 3) + c4) =
-                make_uint2(pack2h(m[0], m[1]), pack2h(m[2], m[3]));
-          }
-        } else {
-#pragma unroll
-          for (int j = 0; j < FN; ++j) {
-            const int col = j * 32 + 8 * q + c4;
-            float v[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              v[e] = acc[i][j][4 * q + e];
-              if constexpr (EPI == kEpiBias) {
-                const int64_t n = tile_n * BN + wn * WC + col + e;
-                v[e] += h2f_bits(g.bias[n < g.N ? n : g.N - 1]);
-              }
-            }
-            *reinterpret_cast<uint2*>(base + stage_off(row, col >> 3) + c4) =
-                make_uint2(pack2h(v[0], v[1]), pack2h(v[2], v[3]));
+        for (int e = 0; e < 4; ++e) {
+          v[e] = acc.get(i, q, e);
+          if constexpr (swiglu_epi(EPI)) {
+            const float gt = h2f(f2h(v[e])), up = h2f(f2h(acc.get(i, q + CG / 2, e)));
+            v[e] = gt * sigmoid_fast(gt) * up;  // as glu_fwd_kernel
+          } else if constexpr (EPI == kEpiBias) {
+            const int64_t n = tile_n * BN + wn * WC + col + e;
+            v[e] += h2f_bits(g.bias[n < g.N ? n : g.N - 1]);
           }
         }
+        *reinterpret_cast<uint2*>(base + stage_off(row, col >> 3) + (col & 7)) =
+            make_uint2(pack2h(v[0], v[1]), pack2h(v[2], v[3]));
       }
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the wavefront's own LDS stores
@@ -587,40 +615,42 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, f32x16 (&acc)[BM /
       if (m < g.M && n < g.N)
         *reinterpret_cast<uint4*>(static_cast<uint16_t*>(g.c) + m * g.ldc + n) = v;
     }
-  } else if constexpr (EPI == kEpiF32) {
-    // fp32 out = alpha acc (+ row-scaled resid), from the registers: each store instruction
-    // writes 32 consecutive columns of two rows; each element's resid is read by the thread
-    // that writes it (out may be resid itself)
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t m = m0 + wm * WR + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-        if (m >= g.M) continue;
-        const float rs = g.resid == nullptr ? 0.0f : g.row_scale == nullptr ? 1.0f
-                                                                              : g.row_scale[m];
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const int64_t n = tile_n * BN + wn * WC + j * 32 + col_in;
-          if (n >= g.N) continue;
-          float v = g.alpha * acc[i][j][r];
-          if (g.resid != nullptr) v += rs * g.resid[m * g.ldr + n];
-          static_cast<float*>(g.c)[m * g.ldc + n] = v;
-        }
-      }
-    }
   } else {
+    // fp32, from the registers, four columns a lane: split-K partials, or out = alpha acc (+
+    // row-scaled resid; each element's resid is read by the thread that writes it: out may be
+    // resid itself). kEpiF32's rows are stored in 16-byte pieces where their alignment allows.
+    float* const out = static_cast<float*>(g.c);
+    const bool wide = EPI == kEpiPartial || g.wide;
 #pragma unroll
-    for (int i = 0; i < FM; ++i) {
+    for (int i = 0; i < RB; ++i) {
+      const int64_t m = m0 + wm * WR + Acc::row(i, lane);
+      if (m >= g.M) continue;
+      float* const orow = EPI == kEpiPartial ? out + ((int64_t)slice * g.M + m) * g.N
+                                             : out + m * g.ldc;
+      const bool has_res = EPI == kEpiF32 && g.resid != nullptr;
+      const float rs = !has_res ? 0.0f : g.row_scale == nullptr ? 1.0f : g.row_scale[m];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t m = m0 + wm * WR + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-        if (m >= g.M) continue;
+      for (int q = 0; q < CG; ++q) {
+        const int64_t n = tile_n * BN + wn * WC + Acc::col(q, lane);
+        if (n >= g.N) continue;  // N % 4 == 0: the four columns lie on one side
+        float v[4];
 #pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const int64_t n = tile_n * BN + wn * WC + j * 32 + col_in;
-          if (n >= g.N) continue;
-          static_cast<float*>(g.c)[((int64_t)slice * g.M + m) * g.N + n] = acc[i][j][r];
+        for (int e = 0; e < 4; ++e) {
+          v[e] = acc.get(i, q, e);
+          if constexpr (EPI == kEpiF32) v[e] *= g.alpha;
+        }
+        if (wide) {
+          if (has_res) {
+            const float4 r = *reinterpret_cast<const float4*>(g.resid + m * g.ldr + n);
+            v[0] += rs * r.x; v[1] += rs * r.y; v[2] += rs * r.z; v[3] += rs * r.w;
+          }
+          *reinterpret_cast<float4*>(orow + n) = make_float4(v[0], v[1], v[2], v[3]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if (has_res) v[e] += rs * g.resid[m * g.ldr + n + e];
+            orow[n + e] = v[e];
+          }
         }
       }
     }
@@ -707,11 +737,11 @@ __global__ __launch_bounds__(kThreads, 1) void nf4_gemm_kernel(GemmArgs g) {
   // vector-memory instructions one k-tile issues (the A DMA, codes and scales)
   constexpr int kVmPerTile = 4 + 2;
 
-  f32x16 acc[4][4];
+  Acc32<4, 4> acc;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x16{};
+    for (int j = 0; j < 4; ++j) acc.a[i][j] = f32x16{};
 
   auto clamp_kt = [&](int64_t kt) { return kt < kt1 ? kt : kt_last; };
   auto issue_tile = [&](int64_t kt, uint16_t* sa, uint16_t* sb) {
@@ -781,7 +811,7 @@ __global__ __launch_bounds__(kThreads, 1) void nf4_gemm_kernel(GemmArgs g) {
     read_frags<NN>(f1, sa, sb, 1, wm, wn, lane);
     nf4_decode_part<NN, NN || decltype(fresh)::value>(c_dec, s_dec, planes, sb_dec, b_row,
                                                       b_chunk0, lv, 0);
-    mfma_step<kT>(acc, f0);
+    mfma_step(acc, f0);
     sched_step<NN, kValu, 0>();
     __builtin_amdgcn_sched_barrier(0);
     sync_tile<kVmPerTile>();  // k-tile t + 1 landed; t + 2 may still be in flight
@@ -793,7 +823,7 @@ __global__ __launch_bounds__(kThreads, 1) void nf4_gemm_kernel(GemmArgs g) {
     nf4_decode_part<NN>(c_dec, s_dec, planes, sb_dec, b_row, b_chunk0, lv, 1);
     c_next = *reinterpret_cast<const uint4*>(c_read + 16 * tid);
     s_next = s_read[tid];
-    mfma_step<kT>(acc, f1);
+    mfma_step(acc, f1);
     sched_step<NN, kValu, kVmPerTile>();
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -822,13 +852,15 @@ __global__ __launch_bounds__(kThreads, 1) void nf4_gemm_kernel(GemmArgs g) {
 // stages per operand; the loop runs one k-tile ahead, each k-tile's DMA instructions spread over
 // three k-steps of the one before.
 //
-// Two tile shapes share the code: 256 x 256 (4 wavefronts of 128 x 128, one workgroup per CU,
-// 128 KB of LDS) for the wide products, and 128 x 128 (4 wavefronts of 64 x 64, 64 KB of LDS, so
-// two workgroups share a CU and cover each other's waits) for the narrow ones (N = 1536 - 2048
-// at a few thousand tokens: 60 tiles of 256 x 256 for 256 CUs, 240 of 128 x 128). A 64 x 64
-// wavefront block reads twice the LDS bytes per MFMA of a 128 x 128 one.
+// Two tile shapes: 256 x 256 (4 wavefronts of 128 x 128, one workgroup per CU, 160 KB of LDS;
+// hgemm256_kernel below) for the wide products, and 128 x 128 (hgemm_kernel: 4 wavefronts of
+// 64 x 64, 64 KB of LDS, so two workgroups share a CU and cover each other's waits) for the narrow
+// ones (N = 1536 - 2048 at a few thousand tokens: 60 tiles of 256 x 256 for 256 CUs, 240 of
+// 128 x 128). A 64 x 64 wavefront block reads twice the LDS bytes per MFMA of a 128 x 128 one. The
+// DMA goes through buffer resources: a 32-bit lane offset is all a load needs (with 64-bit lane
+// addresses the sums cost a VALU instruction a load; [310, 1536] x [17920, 1536] SwiGLU 28.2 ->
+// 25.6 us).
 constexpr int kBK64 = 64;
-constexpr int kTile64 = 256 * kBK64;  // halves per operand stage of a 256 x 256 tile (32 KB)
 
 // [rows][64]: chunk c of row r in slot c ^ ((r >> 1) & 7). A 16-lane group of a fragment read
 // takes 16 consecutive rows of one chunk: two rows per 256-byte bank cycle, eight slots.
@@ -860,9 +892,9 @@ struct DmaKT {
   }
   __device__ __forceinline__ void issue(const uint16_t* base, uint16_t* dst, int wave,
                                         int j) const {
-    __builtin_amdgcn_global_load_lds(reinterpret_cast<const char*>(base) + off[j],
-                                     (lds_void_t*)(dst + ((ROWS / 4) * wave + 8 * j) * 64), 16,
-                                     0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        make_rsrc(base, 0xFFFFFFFFu), (lds_void_t*)(dst + ((ROWS / 4) * wave + 8 * j) * 64), 16,
+        off[j], 0, 0, 0);
   }
 };
 
@@ -882,8 +914,9 @@ struct DmaNT {
   }
   __device__ __forceinline__ void issue(const uint16_t* base, uint16_t* dst, int wave,
                                         int j) const {
-    __builtin_amdgcn_global_load_lds(reinterpret_cast<const char*>(base) + off[j],
-                                     (lds_void_t*)(dst + (16 * wave + RPI * j) * BN), 16, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        make_rsrc(base, 0xFFFFFFFFu), (lds_void_t*)(dst + (16 * wave + RPI * j) * BN), 16, off[j],
+        0, 0, 0);
   }
 };
 
@@ -931,32 +964,17 @@ __device__ __forceinline__ void read_frags64(FragsT<BM / 64, BN / 64>& f, const 
 }
 
 // Tail split, slice partials: the tile's accumulators as fp32 [BM rows][BN B columns] (B column:
-// the tile's n (SwiGLU: its gate and up rows) as the wavefront blocks hold them:
-// wn BN/2 + 32 j + column within the MFMA block). T: transposed accumulators (mfma_step).
-template <bool T, int BM, int BN>
-__device__ __forceinline__ void store_tail_part(float* p, const f32x16 (&acc)[BM / 64][BN / 64],
-                                                int lane, int wave) {
-  constexpr int FM = BM / 64, FN = BN / 64;
+// the tile's n; SwiGLU: its gate and up rows as the wavefront blocks hold them).
+template <int BM, int BN, typename Acc>
+__device__ __forceinline__ void store_tail_part(float* p, const Acc& acc, int lane, int wave) {
   const int wm = wave >> 1, wn = wave & 1;
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
+  for (int i = 0; i < Acc::RB; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      if constexpr (T) {  // register 4 q + e: row i 32 + l % 32, column 8 q + 4 (l / 32) + e
-        float* row = p + (wm * (BM / 2) + i * 32 + (lane & 31)) * BN + wn * (BN / 2) + j * 32 +
-                     4 * (lane >> 5);
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          *reinterpret_cast<float4*>(row + 8 * q) =
-              make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
-                          acc[i][j][4 * q + 3]);
-      } else {  // register r: row i 32 + 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          p[(wm * (BM / 2) + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * BN +
-            wn * (BN / 2) + j * 32 + (lane & 31)] = acc[i][j][r];
-      }
-    }
+    for (int q = 0; q < Acc::CG; ++q)
+      *reinterpret_cast<float4*>(p + (wm * (BM / 2) + Acc::row(i, lane)) * BN + wn * (BN / 2) +
+                                 Acc::col(q, lane)) =
+          make_float4(acc.get(i, q, 0), acc.get(i, q, 1), acc.get(i, q, 2), acc.get(i, q, 3));
 }
 
 // The GEMM with an fp16 B in memory (qlora_gemm16): for 256 x 256 tiles the same wavefront blocks,
@@ -974,8 +992,7 @@ __device__ __forceinline__ void hgemm_tile(const GemmArgs& g, int64_t tile_m, in
                                            uint16_t* sA1, uint16_t* sB0, uint16_t* sB1,
                                            uint16_t* sA2, uint16_t* sA3, uint16_t* sB2,
                                            uint16_t* sB3) {
-  static_assert(BM == BN && (BM == 256 || BM == 128), "square 256 or 128 tiles");
-  static_assert(STAGES == 2 || (STAGES == 4 && BM == 128), "four stages fit 128 x 128 tiles");
+  static_assert(BM == 128 && BN == 128 && (STAGES == 2 || STAGES == 4), "128 x 128 tiles");
   constexpr int FM = BM / 64, FN = BN / 64;
   // DMA instructions a wavefront issues per k-tile (A and B alternate), and how they are dealt:
   // kSA during k-step 3 of the k-tile two before, kSB during k-step 0 of the one before, the rest
@@ -1021,11 +1038,11 @@ __device__ __forceinline__ void hgemm_tile(const GemmArgs& g, int64_t tile_m, in
     b_step = kBK64;
   }
 
-  f32x16 acc[FM][FN];
+  Acc32<FM, FN> acc;
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
+    for (int j = 0; j < FN; ++j) acc.a[i][j] = f32x16{};
 
   // DMA instructions q0 .. q1 - 1 of k-tile kt (q even: A row group q / 2, odd: B's); past the
   // last k-tile the last one is re-read into a stage no longer read
@@ -1056,22 +1073,22 @@ __device__ __forceinline__ void hgemm_tile(const GemmArgs& g, int64_t tile_m, in
       __builtin_amdgcn_sched_barrier(0);
       issue_part(t + 1, sa_n, sb_n, kSA, kSA + kSB);
       read_frags64<NN, BM, BN, TA>(f1, sa, sb, 1, wm, wn, lane);
-      mfma_step<kT>(acc, f0);
+      mfma_step(acc, f0);
       sched_step<NN, 0, kSB, FM, FN, TA>();
       __builtin_amdgcn_sched_barrier(0);
       issue_part(t + 1, sa_n, sb_n, kSA + kSB, kQ);
       read_frags64<NN, BM, BN, TA>(f0, sa, sb, 2, wm, wn, lane);
-      mfma_step<kT>(acc, f1);
+      mfma_step(acc, f1);
       sched_step<NN, 0, kQ - kSA - kSB, FM, FN, TA>();
       __builtin_amdgcn_sched_barrier(0);
       read_frags64<NN, BM, BN, TA>(f1, sa, sb, 3, wm, wn, lane);
-      mfma_step<kT>(acc, f0);
+      mfma_step(acc, f0);
       sched_step<NN, 0, 0, FM, FN, TA>();
       __builtin_amdgcn_sched_barrier(0);
       sync_tile<0>();
       issue_part(t + 2, sa, sb, 0, kSA);
       read_frags64<NN, BM, BN, TA>(f0, sa_n, sb_n, 0, wm, wn, lane);
-      mfma_step<kT>(acc, f1);
+      mfma_step(acc, f1);
       sched_step<NN, 0, kSA, FM, FN, TA>();
       __builtin_amdgcn_sched_barrier(0);
     };
@@ -1095,22 +1112,22 @@ __device__ __forceinline__ void hgemm_tile(const GemmArgs& g, int64_t tile_m, in
       __builtin_amdgcn_sched_barrier(0);
       issue_part(t + 3, sa_p, sb_p, 0, q1);
       read_frags64<NN, BM, BN, TA>(f1, sa, sb, 1, wm, wn, lane);
-      mfma_step<kT>(acc, f0);
+      mfma_step(acc, f0);
       sched_step<NN, 0, q1, FM, FN, TA>();
       __builtin_amdgcn_sched_barrier(0);
       issue_part(t + 3, sa_p, sb_p, q1, q2);
       read_frags64<NN, BM, BN, TA>(f0, sa, sb, 2, wm, wn, lane);
-      mfma_step<kT>(acc, f1);
+      mfma_step(acc, f1);
       sched_step<NN, 0, q2 - q1, FM, FN, TA>();
       __builtin_amdgcn_sched_barrier(0);
       issue_part(t + 3, sa_p, sb_p, q2, kQ);
       read_frags64<NN, BM, BN, TA>(f1, sa, sb, 3, wm, wn, lane);
-      mfma_step<kT>(acc, f0);
+      mfma_step(acc, f0);
       sched_step<NN, 0, kQ - q2, FM, FN, TA>();
       __builtin_amdgcn_sched_barrier(0);
       sync_tile<2 * kQ>();  // t + 1 landed; t + 2, t + 3 may be in flight
       read_frags64<NN, BM, BN, TA>(f0, sa_n, sb_n, 0, wm, wn, lane);
-      mfma_step<kT>(acc, f1);
+      mfma_step(acc, f1);
       sched_step<NN, 0, 0, FM, FN, TA>();
       __builtin_amdgcn_sched_barrier(0);
     };
@@ -1123,7 +1140,7 @@ __device__ __forceinline__ void hgemm_tile(const GemmArgs& g, int64_t tile_m, in
   }
   __builtin_amdgcn_s_waitcnt(0);
   if constexpr (TAIL) {
-    store_tail_part<kT, BM, BN>(g.tail_ws + (int64_t)tail_u * BM * BN, acc, lane, wave);
+    store_tail_part<BM, BN>(g.tail_ws + (int64_t)tail_u * BM * BN, acc, lane, wave);
   } else {
     if constexpr (kT) __builtin_amdgcn_s_barrier();
     // each wavefront stages its fp16 block in one of the four operand stages
@@ -1133,11 +1150,11 @@ __device__ __forceinline__ void hgemm_tile(const GemmArgs& g, int64_t tile_m, in
   }
 }
 
-// STAGES: 2 (either tile; 128 x 128 tiles then leave room for a second workgroup per CU) or 4
-// (128 x 128 only, 128 KB: one workgroup per CU, loads issued three k-tiles ahead).
-template <bool NN, int EPI, int BM, int STAGES, bool TA = false>
-__global__ __launch_bounds__(kThreads, (BM == 128 && STAGES == 2) ? 2 : 1) void hgemm_kernel(
-    GemmArgs g) {
+// 128 x 128 tiles. STAGES: 2 (64 KB of LDS: two workgroups per CU) or 4 (128 KB: one workgroup per
+// CU, loads issued three k-tiles ahead).
+template <bool NN, int EPI, int STAGES, bool TA = false>
+__global__ __launch_bounds__(kThreads, STAGES == 2 ? 2 : 1) void hgemm_kernel(GemmArgs g) {
+  constexpr int BM = 128;
   constexpr int kX = STAGES == 4 ? BM * kBK64 : 8;  // stages 2-3 (unused with two stages)
   __shared__ __attribute__((aligned(1024))) uint16_t sA0[BM * kBK64];
   __shared__ __attribute__((aligned(1024))) uint16_t sA1[BM * kBK64];
@@ -1150,13 +1167,12 @@ __global__ __launch_bounds__(kThreads, (BM == 128 && STAGES == 2) ? 2 : 1) void 
   // past the main tiles: one K slice of one of the last round's tiles (tail split)
   const int tail_u = g.tail_splits > 0 ? (int)blockIdx.x - g.main_tiles : -1;
   if (tail_u >= 0) {
-    const int t = g.main_tiles + tail_u / g.tail_splits;
+    int tm, tn;
+    tile_pos(g.main_tiles + tail_u / g.tail_splits, g.m_tiles, g.tiles / g.m_tiles, tm, tn);
     const int64_t kt0 =
         (int64_t)__builtin_amdgcn_readfirstlane(tail_u % g.tail_splits) * g.kt_per_tail;
-    hgemm_tile<NN, TA, EPI, true, BM, BM, STAGES>(
-        g, __builtin_amdgcn_readfirstlane(t % g.m_tiles),
-        __builtin_amdgcn_readfirstlane(t / g.m_tiles), kt0, kt0 + g.kt_per_tail, tail_u, sA0,
-        sA1, sB0, sB1, sA2, sA3, sB2, sB3);
+    hgemm_tile<NN, TA, EPI, true, BM, BM, STAGES>(g, tm, tn, kt0, kt0 + g.kt_per_tail, tail_u,
+                                                  sA0, sA1, sB0, sB1, sA2, sA3, sB2, sB3);
     return;
   }
   int64_t tile_m, tile_n;
@@ -1166,6 +1182,284 @@ __global__ __launch_bounds__(kThreads, (BM == 128 && STAGES == 2) ? 2 : 1) void 
   const int64_t kt0 = (int64_t)slice * g.kt_per_split;
   hgemm_tile<NN, TA, EPI, false, BM, BM, STAGES>(g, tile_m, tile_n, kt0, kt0 + g.kt_per_split,
                                                  slice, sA0, sA1, sB0, sB1, sA2, sA3, sB2, sB3);
+}
+
+// ---- 256 x 256 tiles ----------------------------------------------------------------------------
+// Four wavefronts of 128 x 128 (one per SIMD), k-tiles of 64 in two k-steps of 32, each 8 x 8
+// v_mfma_f32_16x16x32_f16. On large products the chip's power limit sets the clock (1.5 - 1.9 GHz
+// of 2.4, lower the busier the matrix cores are), so what counts is the work per joule as much as
+// the schedule. A 16x16x32 reads and writes its accumulators once per 32 k, a 32x32x16 twice for
+// the same products (and the same bits: one 16x16x32 equals two 32x32x16 in turn on every one of
+// 2 million random sums): [8192, 8192]^2 826 -> 782 us, the [4001, 3584] x [37888, 3584] SwiGLU
+// product 936 -> 884, with the rest of the kernel the same.
+//
+// The schedule keeps everything else out of the MFMAs' way: every instruction of a k-tile is
+// pinned behind one of its 128 MFMAs (sched_barrier), a fragment read behind every fourth, a DMA
+// behind every eighth (the texture unit takes 64 cycles for the four wavefronts' DMA instructions,
+// an MFMA 16: bunched, they back up and hold the wavefronts' issue). LDS, all 160 KB of the CU:
+// two A stages and three B stages of 32 KB, so that a k-tile's DMA has at least half a k-tile
+// (A) or a whole one (B) to land; with two stages of each and the DMA bunched the [8192, 8192]^2
+// product took 923 us instead of 826 (32x32x16). The DMA is inline assembly: the compiler
+// otherwise holds every LDS read of a dynamically chosen stage behind the DMA in flight; the
+// waits are sync_tile's.
+constexpr uint32_t kStageBytes = 256 * kBK64 * 2;  // of one operand stage
+constexpr uint32_t kLds256 = 5 * kStageBytes;
+
+typedef __attribute__((address_space(3))) const half8_t lds_half8_t;
+
+// One DMA instruction (16 bytes a lane) to LDS byte lds (wave-uniform) + 1024 J + 16 lane. The
+// caller waits for it (sync_tile).
+template <int J>
+__device__ __forceinline__ void dma16(rsrc_t r, uint32_t voff, uint32_t lds) {
+  asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds"
+               :
+               : "s"(lds), "n"(1024 * J), "v"(voff), "s"(r)
+               : "scc");
+}
+
+// acc += a b in place: in assembly, since with all 256 accumulation registers taken the compiler
+// gives some products another destination and copies them back (NN and transposed A). It then
+// does not see the product's latency either: settle() before anything else reads acc. (In the
+// loop 63 others lie between two products of one accumulator.)
+__device__ __forceinline__ void mfma16(f32x4& acc, half8_t a, half8_t b) {
+  asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void settle(Acc16& acc) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    asm volatile("s_nop 15"
+                 : "+a"(acc.a[i][0]), "+a"(acc.a[i][1]), "+a"(acc.a[i][2]), "+a"(acc.a[i][3]),
+                   "+a"(acc.a[i][4]), "+a"(acc.a[i][5]), "+a"(acc.a[i][6]), "+a"(acc.a[i][7]));
+}
+
+// f(0), f(1), .. f(N - 1), each index a compile-time constant.
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void static_for(F f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(f);
+  }
+}
+
+// [64][256] (N-contiguous): chunk c of row k in slot c ^ ((k & 3) << 2) ^ ((k >> 3) & 1) << 1. A
+// half-wavefront's ds_read_b64_tr_b16 takes rows k .. k + 3 and k + 8 .. k + 11 of the same 16
+// columns: eight row pieces of 32 bytes on distinct banks.
+__device__ __forceinline__ int nmaj256_off(int row, int chunk) {
+  return row * 256 + ((chunk ^ ((row & 3) << 2) ^ (((row >> 3) & 1) << 1)) << 3);
+}
+
+// The main loop: k-tiles kt0 .. kt0 + nk - 1 of one tile. NN: B N-contiguous; TA: A M-contiguous
+// (as hgemm_tile).
+template <bool NN, bool TA>
+struct Loop256 {
+  uint32_t offa[8], offb[8];  // lane byte offsets of a wavefront's 8 DMA instructions
+  uint32_t fa[2], fb[2];      // lane LDS addresses of a stage's fragments, by k-step
+  uint32_t wlds;              // LDS byte of the wavefront's 8 KB of stage 0
+  uint32_t sa, sb, sb_n, sb_p;  // stages of this k-tile (A, B) and of the next two (B)
+  rsrc_t ra, rb;
+  const uint16_t *pa, *pb;    // the wavefront's operand rows at the k-tile whose DMA is next
+  uint32_t na, nb;            // their extents in bytes
+  int64_t a_step, b_step;     // elements per k-tile
+  int left;                   // k-tiles after that one
+  int lane, wave;
+  FragsT<8, 8> f0, f1;
+
+  // Rows past M (or past N, NT's last tile) lie past the resources' extents: they are not read,
+  // and their products are not stored.
+  template <int EPI>
+  __device__ __forceinline__ void init(const GemmArgs& g, int tile_m, int tile_n, int kt0, int nk,
+                                       uint16_t* smem) {
+    const int tid = threadIdx.x;
+    lane = tid & 63;
+    wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void_t*)smem;
+    wlds = lds0 + 8192u * wave;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      // K-contiguous: rows 8 j + lane / 8 of the wavefront's 64, swizzled as kmaj64_off;
+      // N-contiguous: k-rows 2 j + lane / 32 of its 16, as nmaj256_off
+      const uint32_t rk = 8 * j + (lane >> 3), ck = (lane & 7) ^ ((rk >> 1) & 7);
+      const uint32_t rn = 2 * j + (lane >> 5),
+                     cn = (lane & 31) ^ ((rn & 3) << 2) ^ (((rn >> 3) & 1) << 1);
+      offa[j] = TA ? (rn * (uint32_t)g.lda + 8 * cn) * 2 : (rk * (uint32_t)g.lda + 8 * ck) * 2;
+      offb[j] = NN ? (rn * (uint32_t)g.ldb + 8 * cn) * 2 : (rk * (uint32_t)g.ldb + 8 * ck) * 2;
+    }
+    a_step = TA ? (int64_t)kBK64 * g.lda : kBK64;
+    b_step = NN ? (int64_t)kBK64 * g.ldb : kBK64;
+    // fragment of 16 rows (columns) x 32 k: lane l holds row l % 16, k 8 (l / 16) .. + 7
+    const int p = lane & 15, q = lane >> 4;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int k = 32 * s + 8 * q + (p >> 2);  // ds_read_b64_tr_b16: as read_frag_tr
+      fa[s] = lds0 + 2 * (TA ? nmaj256_off(k, (wm * 128 + 4 * (p & 3)) >> 3) + 4 * (p & 1)
+                             : kmaj64_off(wm * 128 + p, 4 * s + q));
+      fb[s] = lds0 + 2 * (NN ? nmaj256_off(k, (wn * 128 + 4 * (p & 3)) >> 3) + 4 * (p & 1)
+                             : kmaj64_off(wn * 128 + p, 4 * s + q));
+    }
+    sa = 0;
+    sb = 2 * kStageBytes;
+    sb_n = 3 * kStageBytes;
+    sb_p = 4 * kStageBytes;
+
+    const int64_t m0 = (int64_t)tile_m * 256, k0 = (int64_t)kt0 * kBK64;
+    if constexpr (TA) {  // whole tiles of M (host check)
+      pa = g.a + (k0 + 16 * wave) * g.lda + m0;
+      na = 0xFFFFFFFFu;
+    } else {
+      const int64_t rows = g.M - m0 - 64 * wave;
+      pa = g.a + (rows > 0 ? m0 + 64 * wave : 0) * g.lda + k0;
+      na = (uint32_t)((rows < 0 ? 0 : rows > 64 ? 64 : rows) * g.lda * 2);
+    }
+    if constexpr (NN) {
+      pb = g.b + (k0 + 16 * wave) * g.ldb + (int64_t)tile_n * 256;
+      nb = 0xFFFFFFFFu;
+    } else {
+      const int64_t row = nt_wrow<EPI, 256>(g, tile_n, 64 * wave);
+      const int64_t rows = swiglu_epi(EPI) ? 64 : g.N - row;
+      pb = g.b + (rows > 0 ? row : 0) * g.ldb + k0;
+      nb = (uint32_t)((rows < 0 ? 0 : rows > 64 ? 64 : rows) * g.ldb * 2);
+    }
+    left = nk - 1;
+  }
+  // On to the next k-tile; past the last one that is loaded again, into a stage no longer read.
+  __device__ __forceinline__ void next() {
+    if (left > 0) {
+      pa += a_step;
+      pb += b_step;
+    }
+    --left;
+  }
+
+  template <int J0, int J1>
+  __device__ __forceinline__ void dma_a(uint32_t stage) {
+    static_for<J1 - J0>([&](auto j) { dma16<J0 + j.value>(ra, offa[J0 + j.value], wlds + stage); });
+  }
+  template <int J0, int J1>
+  __device__ __forceinline__ void dma_b(uint32_t stage) {
+    static_for<J1 - J0>([&](auto j) { dma16<J0 + j.value>(rb, offb[J0 + j.value], wlds + stage); });
+  }
+
+  // Fragment read R (0 .. 15: B's eight blocks, then A's) of k-step S. Block i of an operand is 16
+  // rows on (K-contiguous: 2,048 bytes) or 16 columns on (N-contiguous: two chunks, which the
+  // swizzle moves within 16 chunks by XOR: an XOR of 32 i bytes).
+  template <int S, int R>
+  __device__ __forceinline__ void read(FragsT<8, 8>& f, uint32_t st_a, uint32_t st_b) {
+    constexpr int i = R & 7;
+    if constexpr (R < 8)
+      f.b[i] = NN ? tr_frag((fb[S] ^ (32u * i)) + st_b)
+                  : *(lds_half8_t*)(uintptr_t)(fb[S] + st_b + 2048u * i);
+    else
+      f.a[i] = TA ? tr_frag((fa[S] ^ (32u * i)) + st_a)
+                  : *(lds_half8_t*)(uintptr_t)(fa[S] + st_a + 2048u * i);
+  }
+  // rows k .. k + 3 and k + 4 .. k + 7 of an N-contiguous stage (512 bytes a row), transposed
+  static __device__ __forceinline__ half8_t tr_frag(uint32_t addr) {
+    const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(uintptr_t)addr);
+    const short4_t hi =
+        __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(uintptr_t)(addr + 4 * 512));
+    return __builtin_bit_cast(half8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  }
+
+  // The DMA of the first two k-tiles and the first fragments.
+  __device__ __forceinline__ void prologue() {
+    ra = make_rsrc(pa, na);
+    rb = make_rsrc(pb, nb);
+    dma_a<0, 8>(sa);
+    dma_b<0, 8>(sb);
+    next();
+    ra = make_rsrc(pa, na);
+    rb = make_rsrc(pb, nb);
+    dma_b<0, 8>(sb_n);
+    dma_a<0, 8>(sa ^ kStageBytes);
+    sync_tile<16>();  // the first k-tile landed
+    static_for<16>([&](auto r) { read<0, r.value>(f0, sa, sb); });
+  }
+
+  // 32 of a k-step's 64 MFMAs (rows 4 H .. 4 H + 3 of blocks) on fragments fc, eight reads of
+  // k-step SN into fn and four DMA instructions among them.
+  template <int H, int SN, typename Dma>
+  __device__ __forceinline__ void half_step(Acc16& acc, const FragsT<8, 8>& fc, FragsT<8, 8>& fn,
+                                            uint32_t st_a, uint32_t st_b, Dma dma) {
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<32>([&](auto qc) {
+      constexpr int q = qc.value, i = 4 * H + (q >> 3), j = q & 7;
+      mfma16(acc.a[i][j], fc.b[j], fc.a[i]);
+      if constexpr ((q & 3) == 0) read<SN, 8 * H + (q >> 2)>(fn, st_a, st_b);
+      if constexpr ((q & 7) == 2) dma(std::integral_constant<int, (q >> 3)>{});
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  }
+
+  // One k-tile (t). Its first k-step reads its second's fragments and starts B's DMA of t + 2
+  // (into the stage of t - 1). Then every wavefront has read this k-tile's stages and t + 1 has
+  // landed (the barrier: only t + 2's B is younger); the second k-step reads t + 1's first
+  // fragments and starts A's DMA of t + 2 into this k-tile's stage.
+  __device__ __forceinline__ void k_tile(Acc16& acc) {
+    const uint32_t sa_n = sa ^ kStageBytes;
+    // the blocks' addresses are formed in the k-tile that uses them: hoisted out of the loop they
+    // would take more registers than the accumulators leave
+    asm volatile("" : "+v"(fa[0]), "+v"(fa[1]), "+v"(fb[0]), "+v"(fb[1]));
+    next();
+    rb = make_rsrc(pb, nb);
+    half_step<0, 1>(acc, f0, f1, sa, sb, [&](auto j) { dma_b<j.value, j.value + 1>(sb_p); });
+    half_step<1, 1>(acc, f0, f1, sa, sb, [&](auto j) { dma_b<4 + j.value, 5 + j.value>(sb_p); });
+    ra = make_rsrc(pa, na);
+    sync_tile<8>();
+    half_step<0, 0>(acc, f1, f0, sa_n, sb_n, [&](auto j) { dma_a<j.value, j.value + 1>(sa); });
+    half_step<1, 0>(acc, f1, f0, sa_n, sb_n, [&](auto j) { dma_a<4 + j.value, 5 + j.value>(sa); });
+    sa = sa_n;
+    const uint32_t x = sb;
+    sb = sb_n;
+    sb_n = sb_p;
+    sb_p = x;
+  }
+};
+
+// One 256 x 256 tile (or one K slice of it: TAIL as hgemm_tile) over k-tiles kt0 .. kt1 - 1.
+template <bool NN, bool TA, int EPI, bool TAIL>
+__device__ __forceinline__ void hgemm256_tile(const GemmArgs& g, int tile_m, int tile_n, int kt0,
+                                              int kt1, int tail_u, uint16_t* smem) {
+  const int ktiles = (int)(g.Kr / kBK64);
+  if (kt1 > ktiles) kt1 = ktiles;
+  Loop256<NN, TA> lp;
+  lp.template init<EPI>(g, tile_m, tile_n, kt0, kt1 - kt0, smem);
+  Acc16 acc;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc.a[i][j] = f32x4{};
+  lp.prologue();
+  settle(acc);
+  for (int t = kt0; t < kt1; ++t) lp.k_tile(acc);
+  __builtin_amdgcn_s_waitcnt(0);
+  settle(acc);
+  if constexpr (TAIL) {
+    store_tail_part<256, 256>(g.tail_ws + (int64_t)tail_u * 65536, acc, lp.lane, lp.wave);
+  } else {
+    if constexpr (staged_epi(EPI)) __builtin_amdgcn_s_barrier();
+    uint16_t* st = smem + lp.wave * (256 * kBK64);  // fp16 outputs: staged in a stage each
+    store_tile<EPI, 256, 256>(g, acc, st, st + 64 * 128, (int64_t)tile_m * 256, tile_n, lp.lane,
+                              lp.wave, tail_u);
+  }
+}
+
+template <bool NN, int EPI, bool TA = false>
+__global__ __launch_bounds__(kThreads, 1) void hgemm256_kernel(GemmArgs g) {
+  __shared__ __attribute__((aligned(1024))) uint16_t smem[kLds256 / 2];
+  const int tail_u = g.tail_splits > 0 ? (int)blockIdx.x - g.main_tiles : -1;
+  if (tail_u >= 0) {
+    int tm, tn;
+    tile_pos(g.main_tiles + tail_u / g.tail_splits, g.m_tiles, g.tiles / g.m_tiles, tm, tn);
+    const int kt0 = __builtin_amdgcn_readfirstlane(tail_u % g.tail_splits) * g.kt_per_tail;
+    hgemm256_tile<NN, TA, EPI, true>(g, tm, tn, kt0, kt0 + g.kt_per_tail, tail_u, smem);
+    return;
+  }
+  int64_t tm, tn;
+  int slice;
+  tile_of(g.m_tiles, g.tiles, g.tail_splits > 0 ? g.main_tiles : (int)gridDim.x, tm, tn, slice);
+  hgemm256_tile<NN, TA, EPI, false>(g, (int)tm, (int)tn, slice * g.kt_per_split,
+                                    (slice + 1) * g.kt_per_split, slice, smem);
 }
 
 // Tail split: the slices of each tail tile summed in slice order, then the epilogue (fp16 store,
@@ -1178,7 +1472,9 @@ __global__ __launch_bounds__(256) void tail_reduce_kernel(GemmArgs g, int epi, i
   if (id >= (int64_t)tiles * per_tile) return;
   const int u = (int)(id / per_tile), w = (int)(id - (int64_t)u * per_tile);
   const int t = g.main_tiles + u;
-  const int64_t tile_m = t % g.m_tiles, tile_n = t / g.m_tiles;
+  int tm, tn;
+  tile_pos_lane(t, g.m_tiles, g.tiles / g.m_tiles, tm, tn);
+  const int64_t tile_m = tm, tile_n = tn;
   const int64_t slice = (int64_t)BM * BN;
   const float* part = g.tail_ws + (int64_t)u * g.tail_splits * slice;
   const int S = g.tail_splits;
@@ -1292,7 +1588,8 @@ template <int BSRC, bool NN, int EPI, int BM, int ST, bool TA = false>
 void launch_one(const GemmArgs& g, dim3 grid, hipStream_t s, hipEvent_t start, hipEvent_t stop) {
   auto kernel = [] {
     if constexpr (BSRC == kBNF4) return nf4_gemm_kernel<NN, EPI>;
-    else return hgemm_kernel<NN, EPI, BM, ST, TA>;
+    else if constexpr (BM == 128) return hgemm_kernel<NN, EPI, ST, TA>;
+    else return hgemm256_kernel<NN, EPI, TA>;
   }();
   if (start != nullptr || stop != nullptr)
     hipExtLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, s, start, stop, 0, g);
@@ -1815,6 +2112,7 @@ QLORA_API int qlora_gemm16_f32(const void* a, int64_t lda, const void* b, int64_
   g.Kr = K;
   g.alpha = alpha;
   g.row_scale = row_scale;
+  g.wide = ldc % 4 == 0 && al(c, 16) && (resid == nullptr || (ldr % 4 == 0 && al(resid, 16)));
   return run_gemm(g, kBHalf, mode, kEpiF32, splits, ws, ws_elems, (hipStream_t)stream, nullptr,
                   nullptr, tile, stages);
 }
