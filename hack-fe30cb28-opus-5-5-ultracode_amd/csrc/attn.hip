@@ -24,9 +24,10 @@
 // LDS tiles are XOR-swizzled by 16-byte chunk so that the operand reads (32 rows, same chunk)
 // and the staging writes are spread over the banks.
 //
-// One workgroup = the q heads that share a kv head (forward, dQ), which share the staged K/V
-// tiles; dK/dV: four wavefronts on 128 consecutive keys of one q head, sharing the staged Q/dO.
-// Global loads of the next tile are issued before the current tile's MFMAs (register
+// One workgroup = consecutive (query tile, q head) pairs of one kv head (forward) or the q heads
+// that share a kv head (dQ), which share the staged K/V tiles; dK/dV: four wavefronts on 128
+// consecutive keys of one q head, sharing the staged Q/dO. The next tile's loads are in flight
+// during the current tile's MFMAs (forward: LDS DMA; dQ, dK/dV: global loads into registers, a
 // prefetch), so their latency overlaps the arithmetic. dK/dV come out per q head
 // ([n, HQ, D]); the caller sums each group (the RoPE backward does, as the reference sums the
 // repeated kv heads). The log-sum-exp of the forward (natural log, fp32 [HQ, n]) and
@@ -87,7 +88,7 @@ __device__ __forceinline__ f32x16 mfma(half8_t a, half8_t b, f32x16 c) {
 
 // [rows][D] tile, 16-byte chunk c of row r at chunk c ^ (r mod D/8).
 template <int D>
-__device__ __forceinline__ int rm_off(int row, int chunk) {
+__host__ __device__ constexpr int rm_off(int row, int chunk) {
   return row * D + ((chunk ^ (row & (D / 8 - 1))) << 3);
 }
 
@@ -95,7 +96,7 @@ __device__ __forceinline__ int rm_off(int row, int chunk) {
 // consecutive rows (the first a multiple of 4) x 4 aligned chunks, which this swizzle spreads
 // over distinct banks; 16-byte row stores (16 threads a row) stay conflict-free too.
 template <int D>
-__device__ __forceinline__ int tt_off(int row, int chunk) {
+__host__ __device__ constexpr int tt_off(int row, int chunk) {
   const int j = D == 128 ? row : row >> 1;  // rows sharing the 64 banks: 1 (D = 128) or 2
   const int sw = D == 128 ? (((j & 3) << 2) | ((j >> 2) & 3)) : (((j & 1) << 2) | ((j >> 1) & 3));
   return row * D + ((chunk ^ sw) << 3);
@@ -233,137 +234,360 @@ __device__ __forceinline__ void store_token_row_f32(float* row, const f32x16 (&a
 
 // ------------------------------------------------------------------------------------------------
 // Forward: O = softmax(scale Q K^T + causal mask) V per sequence, and the log-sum-exp.
-// grid (ceil(max_len / 32) * nseq * KH, 1, chunks), block 64 * G (G = HQ / KH q heads, one per
-// wavefront). Key blocks of 64 keys: block kb + 1 is loaded into registers while block kb is
-// multiplied. The longest query tiles' key ranges set the kernel's time when the batch has few
-// sequences (the rest of the GPU idles): cutting the range into chunks spreads one tile over
-// several workgroups.
+//
+// A workgroup is NW wavefronts, one query tile each: NW consecutive (query tile, q head) pairs of
+// one kv head, the heads fastest, which share the staged K/V blocks of 64 keys. Two wavefronts run
+// per SIMD. The kernel is bound by what the SIMDs issue (per block and wavefront 32 MFMAs, 1,024
+// cycles of the matrix core, beside 130 VALU instructions, 32 of them exponentials), so a block's
+// softmax is formed two values at a time behind the MFMAs of the next block's S and of P V (every
+// instruction pinned behind an MFMA by sched_barrier), no address is formed per fragment
+// (RowFrags, TrFrags), masks are applied from the diagonal on only, and the running maximum is
+// only a reference: it moves (and O is rescaled) when a score exceeds it by more than 2^8, so p <=
+// 2^8 and most blocks never rescale. K and V arrive by LDS DMA, two stages each, one barrier a
+// block. MI355X, 12/2 heads of 128, against one q head group per workgroup with the blocks staged
+// through registers and two barriers a block: four sequences of 283-997 tokens 36 -> 24 us, two of
+// 4,096 and 3,001 165 -> 100.
+// NW 4 or 8: four wavefronts spread a small batch over the CUs (24 us against 31 for those four
+// sequences); once 2,048 tiles fill all of them eight read K and V half as often (4,096 + 3,001,
+// forward and backward: 574 -> 560 us).
+// grid (ceil(ceil(max_len / 32) G / NW) nseq KH, 1, chunks), block 64 NW.
 // ------------------------------------------------------------------------------------------------
-template <int D, int G>
-__global__ __launch_bounds__(64 * G) void attn_fwd_kernel(Args a) {
-  constexpr int KC = D / 16, DT = D / 32, NT = 64 * G;
-  __shared__ __align__(16) uint16_t ks[kKB * D];
-  __shared__ __align__(16) uint16_t vs[kKB * D];
-  // blockIdx.x = tile + ntiles (seq KH + kvh), the tile fastest: consecutive workgroups (which
-  // the dispatcher deals to the 8 XCDs in turn) take tiles of the same sequence, so every XCD
-  // gets a share of each; the longest rows first
-  const int sh = blockIdx.x / a.ntiles;
-  const int tile = a.ntiles - 1 - (int)(blockIdx.x - sh * a.ntiles);
+constexpr float kRescale = 8.f;  // log2 units
+
+// max(a, b, c) without the quieting of signalling NaNs that fmaxf adds per operand.
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+// max (sum) of lanes l and l ^ 32
+__device__ __forceinline__ float pair_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                  false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ uint32_t cvt2h(float a, float b) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){a, b}, h2));
+}
+
+// LDS byte addresses of the fragments of a [rows][D] stage. A swizzle acts on chunk bits that the
+// fragment's column offset only flips, so a few lane addresses (one per column offset, formed once
+// a block: N of them) and immediate row offsets reach all of a stage's fragments.
+typedef __attribute__((address_space(3))) const half8_t lds_half8_t;
+// rm_off stage (TT: tt_off): fragment (kk, half): row lane % 32 + 32 half, chunk 2 kk + lane / 32.
+template <int D, bool TT = false>
+struct RowFrags {
+  uint32_t at[D / 16];
+  __device__ __forceinline__ void set(uint32_t stage, int lane) {
+    const uint32_t l0 = (uint32_t)(2 * (TT ? tt_off<D>(lane & 31, lane >> 5) : rm_off<D>(lane & 31, lane >> 5)));
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk) at[kk] = l0 ^ (uint32_t)(32 * kk);
+    move(stage);
+  }
+  __device__ __forceinline__ void move(uint32_t by) {
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk) {
+      at[kk] += by;
+      asm volatile("" : "+v"(at[kk]));  // the row offsets stay immediates
+    }
+  }
+  __device__ __forceinline__ half8_t get(int kk, int half) const {
+    return *(lds_half8_t*)(uintptr_t)(at[kk] + (uint32_t)(half * 32 * D * 2));
+  }
+};
+// tt_off stage read transposed: fragment (kk, u): tokens 16 kk .., columns 32 u .. (tr_operand).
+template <int D>
+struct TrFrags {
+  uint32_t lo[D / 32], hi[D / 32];
+  __device__ __forceinline__ void set(uint32_t stage, int lane) {
+    const int p = lane & 15, col = 16 * ((lane >> 4) & 1) + 4 * (p & 3);
+    const uint32_t l0 =
+        (uint32_t)(2 * (tt_off<D>(4 * (lane >> 5) + (p >> 2), col >> 3) + (col & 7)));
+#pragma unroll
+    for (int u = 0; u < D / 32; ++u) {
+      lo[u] = l0 ^ (uint32_t)(64 * u);
+      hi[u] = l0 ^ (uint32_t)(64 * u + 32);  // eight rows on: two chunks flipped
+    }
+    move(stage);
+  }
+  __device__ __forceinline__ void move(uint32_t by) {
+#pragma unroll
+    for (int u = 0; u < D / 32; ++u) {
+      lo[u] += by;
+      hi[u] += by;
+      asm volatile("" : "+v"(lo[u]), "+v"(hi[u]));
+    }
+  }
+  __device__ __forceinline__ half8_t get(int kk, int u) const {
+    const uint32_t a0 = lo[u] + (uint32_t)(16 * kk * D * 2), a1 = hi[u] + (uint32_t)((16 * kk + 8) * D * 2);
+    const short4_t x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(uintptr_t)a0);
+    const short4_t y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(uintptr_t)a1);
+    return __builtin_bit_cast(half8_t, __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7));
+  }
+};
+
+// The DMA of ROWS-row blocks of a token-major matrix by NW wavefronts (ROWS / NW rows each) into a
+// swizzled [ROWS][D] stage (rm_off, or TT: tt_off).
+template <int D, int ROWS, int NW, bool TT>
+struct BlockDma {
+  static constexpr int CPR = D / 8, RPI = 64 / CPR, RW = ROWS / NW;
+  static constexpr int N = RW / RPI;  // instructions a wavefront
+  static_assert(RW % RPI == 0 && RW <= 16, "whole instructions, rows of one swizzle period");
+  uint32_t off;    // lane byte offset of instruction 0's rows of the block in the sequence
+  uint32_t row_b;  // bytes of one instruction's rows
+  __device__ __forceinline__ void init(int row0, int stride_b, int lane, int wave) {
+    const int r = RW * wave + lane / CPR;
+    const int o = TT ? tt_off<D>(r, lane % CPR) : rm_off<D>(r, lane % CPR);  // XOR: an involution
+    off = (uint32_t)((row0 + r) * stride_b + (o - r * D) * 2);
+    row_b = (uint32_t)(RPI * stride_b);
+  }
+  // Instruction J's rows swizzle as instruction 0's with some chunk bits flipped (an XOR of the
+  // byte offset: the rows themselves are whole multiples of CPR chunks apart).
+  template <int J>
+  static constexpr uint32_t flip() {
+    const int r = RPI * J;  // (RW wave: the flip does not depend on it, RW J' < 16 rows apart)
+    return (uint32_t)(2 * (TT ? tt_off<D>(r, 0) - r * D : rm_off<D>(r, 0) - r * D));
+  }
+  template <int J>
+  __device__ __forceinline__ void issue(rsrc_t src, uint32_t lds, int wave) const {
+    dma16<J>(src, (off ^ flip<J>()) + J * row_b, lds + (uint32_t)(RW * wave * D * 2));
+  }
+  __device__ __forceinline__ void step(uint32_t bytes) {
+    off += bytes;
+    asm volatile("" : "+v"(off));  // the other offsets are formed when they are used
+  }
+};
+
+// Steps of the probabilities done before product q of the ns that form the next block's scores.
+constexpr int p_of(int q, int ns) {
+  return q < ns / 2 ? q * 8 / (ns / 2) : 8 + (q - ns / 2) * 4 / (ns / 2);
+}
+
+template <int D, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void attn_fwd_kernel(Args a) {
+  constexpr int KC = D / 16, DT = D / 32, kStage = kKB * D;
+  typedef BlockDma<D, kKB, NW, false> KDma;
+  typedef BlockDma<D, kKB, NW, true> VDma;
+  constexpr int NI = KDma::N;
+  constexpr int kAhead = 3;  // fragment reads issued ahead of their MFMAs
+  __shared__ __align__(1024) uint16_t smem[4 * kStage];  // two K stages, two V stages
+  const int G = a.HQ / a.KH;
+  // blockIdx.x = rank pairs + (seq KH + kvh - rank) mod pairs: the longest rows of every sequence
+  // first (a late long one would end last), and since the dispatcher deals consecutive workgroups
+  // to the 8 XCDs in turn, a sequence's groups move on by one XCD a rank
+  const int pairs = gridDim.x / a.ntiles, rank = blockIdx.x / pairs;
+  const int sh = ((int)blockIdx.x - rank * pairs + rank) % pairs, grp = a.ntiles - 1 - rank;
   const int seq = sh / a.KH, kvh = sh % a.KH;
-  const int q0 = tile * kTok;
   const int start = a.cu[seq], L = a.cu[seq + 1] - start;
-  if (q0 >= L) return;
+  const int total = (L + kTok - 1) / kTok * G;
+  if (grp * NW >= total) return;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int h = kvh * G + __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
-  const int qi = q0 + (lane & 31);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  auto blocks_of = [&](int f) { return (min(f / G * kTok + kTok, L) + kKB - 1) / kKB; };
+  const int nkb = blocks_of(min(grp * NW + NW - 1, total - 1));  // of the longest tile
+  const int ch = blockIdx.z;
+  if (ch >= num_chunks(nkb, a.chunk)) return;
+  const int kb0 = ch * a.chunk, kb1 = num_chunks(nkb, a.chunk) == 1 ? nkb : min(nkb, kb0 + a.chunk);
+
   const int64_t qs = (int64_t)a.HQ * D, kvs = (int64_t)a.KH * D;
   const int kvs_b = (int)(kvs * 2);
-  const int kend = min(q0 + kTok, L);
-  const int nkb = (kend + kKB - 1) / kKB;
-  const int nch = num_chunks(nkb, a.chunk), ch = blockIdx.z;
-  if (ch >= nch) return;
-  const int kb0 = ch * a.chunk, kb1 = nch == 1 ? nkb : min(nkb, kb0 + a.chunk);
   const rsrc_t ksrc = rows_rsrc(a.k + (int64_t)start * kvs + kvh * D, L, kvs, D);
   const rsrc_t vsrc = rows_rsrc(a.v + (int64_t)start * kvs + kvh * D, L, kvs, D);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
+  KDma kd;
+  VDma vd;
+  kd.init(kb0 * kKB, kvs_b, lane, wave);
+  vd.init(kb0 * kKB, kvs_b, lane, wave);
+  const uint32_t blk_b = (uint32_t)(kKB * kvs_b);
+  // stage s (0, 1) of K and V
+  auto k_lds = [&](int s) { return lds0 + (uint32_t)(s * kStage * 2); };
+  auto v_lds = [&](int s) { return lds0 + (uint32_t)((2 + s) * kStage * 2); };
+  auto dma_k = [&](int s) {
+    static_for<NI>([&](auto j) { kd.template issue<j.value>(ksrc, k_lds(s), wave); });
+    kd.step(blk_b);
+  };
+  dma_k(0);
+  dma_k(1);
+  static_for<NI>([&](auto j) { vd.template issue<j.value>(vsrc, v_lds(0), wave); });
+  vd.step(blk_b);
 
-  RowStage<D, kKB, NT> sk;
-  RowStage<D, kKB, NT, true> sv;
-  sk.load(ksrc, kb0 * kKB, kvs_b, tid);
-  sv.load(vsrc, kb0 * kKB, kvs_b, tid);
-
+  // the wavefront's tile: q head, first query, this lane's query and the last key it attends to;
+  // past the last tile: the last one again, not stored
+  const int f = grp * NW + wave, fc = min(f, total - 1);
+  const int h = kvh * G + __builtin_amdgcn_readfirstlane(fc % G);
+  const int q0 = __builtin_amdgcn_readfirstlane(fc / G) * kTok;
+  const int qi = q0 + (lane & 31), lim = min(qi, L - 1);
+  const int nch = num_chunks(blocks_of(fc), a.chunk);
+  const bool live = f < total && ch < nch;
   half8_t qr[KC];  // queries past the sequence read zeros (their rows are not stored)
   load_token<D>(rows_rsrc(a.q + (int64_t)start * qs + h * D, L, qs, D), qi, (int)(qs * 2), lane,
                 qr);
-  f32x16 o[DT];
+  f32x16 o[DT], s[2], sn[2];
+  half8_t pb[4];
+  float m, mx, lsum = 0.f;
+  const float c = a.scale * kLog2e;
 #pragma unroll
   for (int u = 0; u < DT; ++u) o[u] = f32x16{};
-  float m = -__builtin_inff(), lsum = 0.f;
-  const float c = a.scale * kLog2e;
-  const int lim = min(qi, L - 1);  // the last key this query attends to
 
-  // one key block from the staged tiles (ks, vs)
-  auto block = [&](int k0) {
-    f32x16 s[2];
-    s[0] = s[1] = f32x16{};
+  // K fragment f = half KC + kk (half: of the 64 keys) and V fragment f = kk DT + u of a stage
+  half8_t kf[2 * KC], vf[4 * DT];
+  RowFrags<D> kat;
+  TrFrags<D> vat;
+  kat.set(k_lds(0), lane);
+  vat.set(v_lds(0), lane);
+  auto read_k = [&](auto i) { kf[i.value] = kat.get(i.value % KC, i.value / KC); };
+  auto read_v = [&](auto i) { vf[i.value] = vat.get(i.value / DT, i.value % DT); };
+  // MFMA q of S = K Q^T: fragment q
+  auto s_mfma = [&](auto qc, f32x16 (&x)[2]) {
+    constexpr int kk = qc.value % KC, hf = qc.value / KC;
+    x[hf] = mfma(kf[qc.value], qr[kk], kk == 0 ? f32x16{} : x[hf]);
+  };
+  // a block on the diagonal: keys past the query are masked
+  auto mask = [&](f32x16 (&x)[2], int k0) {
+    const int d = lim - k0 - 4 * (lane >> 5);  // acc_row(r, lane) is acc_row(r, 0) past that
 #pragma unroll
-    for (int kk = 0; kk < KC; ++kk) {
-      const half8_t k0op = ld_rm<D>(ks, lane & 31, 2 * kk + (lane >> 5));
-      const half8_t k1op = ld_rm<D>(ks, 32 + (lane & 31), 2 * kk + (lane >> 5));
-      s[0] = mfma(k0op, qr[kk], s[0]);
-      s[1] = mfma(k1op, qr[kk], s[1]);
-    }
-    if (k0 + kKB - 1 > q0) {  // a block on the diagonal (uniform): mask keys past the query
+    for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          s[t][r] = k0 + 32 * t + acc_row(r, lane) > lim ? -__builtin_inff() : s[t][r];
-    }
-    // the state is in log2 units of the scaled scores: m = max(c s), p = 2^(c s - m)
-    float mx = -__builtin_inff();
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[t][r]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float mnew = fmaxf(m, mx * c);
-    const float alpha = ex2(m - mnew);
-    m = mnew;
-    float ps = 0.f;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float p = ex2(fmaf(s[t][r], c, -mnew));
-        s[t][r] = p;
-        ps += p;
-      }
-    lsum = lsum * alpha + ps;
-    if (__any(alpha != 1.f)) {  // once the running maxima settle, most blocks skip this
+      for (int r = 0; r < 16; ++r)
+        x[hf][r] = 32 * hf + acc_row(r, 0) > d ? -__builtin_inff() : x[hf][r];
+  };
+  // Step i (0 .. 15) of the block's maximum: two values.
+  auto max_step = [&](auto ic, const f32x16 (&x)[2]) {
+    constexpr int hf = ic.value >> 3, r = 2 * (ic.value & 7);
+    mx = max3(ic.value == 0 ? -__builtin_inff() : mx, x[hf][r], x[hf][r + 1]);
+  };
+  // Step i (0 .. 15) of the block's probabilities: two values of P fragment i / 4. The state is in
+  // log2 units of the scaled scores.
+  auto p_step = [&](auto ic, const f32x16 (&x)[2]) {
+    constexpr int kk = ic.value >> 2, e = 2 * (ic.value & 3);
+    const float p0 = ex2(fmaf(x[kk >> 1][8 * (kk & 1) + e], c, -m));
+    const float p1 = ex2(fmaf(x[kk >> 1][8 * (kk & 1) + e + 1], c, -m));
+    lsum += p0 + p1;
+    uint4 w = __builtin_bit_cast(uint4, pb[kk]);
+    (e == 0 ? w.x : e == 2 ? w.y : e == 4 ? w.z : w.w) = cvt2h(p0, p1);
+    pb[kk] = __builtin_bit_cast(half8_t, w);
+  };
+
+  int cur = 0;                                // the stage of K(b) and V(b); b + 1's is the other
+  uint32_t k_at = k_lds(0), v_at = v_lds(0);  // the stages kat and vat address
+  // Block b: its scores (masked) in x and their maximum in mx; the next block's go to xn and mx.
+  // last: there is none; masked: the next block reaches past the first query.
+  auto block = [&](auto last, auto masked, int b, f32x16 (&x)[2], f32x16 (&xn)[2]) {
+    constexpr bool kLast = last.value;
+    const int next = cur ^ 1;
+    constexpr int NS = 2 * KC, NV = 4 * DT;  // MFMAs of S and of P V
+    sync_tile<0>();  // K(b + 1) and V(b) landed, every wavefront is done with b - 1
+    if (!kLast) kat.move(k_lds(next) - k_at);
+    k_at = k_lds(next);
+    vat.move(v_lds(cur) - v_at);
+    v_at = v_lds(cur);
+    if (!kLast) static_for<kAhead>([&](auto i) { read_k(i); });
+    else static_for<kAhead>([&](auto i) { read_v(i); });
+    const bool grow = mx * c > m + kRescale;
+    if (__any(grow)) {
+      const float mn = grow ? mx * c : m;
+      const float alpha = grow ? ex2(m - mn) : 1.0f;
+      m = mn;
+      lsum *= alpha;
 #pragma unroll
       for (int u = 0; u < DT; ++u)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[u][r] *= alpha;
     }
-    half8_t pb[4];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) pb[kk] = to_b(s[kk >> 1], kk & 1);
-#pragma unroll
-    for (int u = 0; u < DT; ++u) {
-      half8_t vop[4];
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) vop[kk] = tr_operand<D>(vs, 16 * kk, 32 * u, lane);
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) o[u] = mfma(vop[kk], pb[kk], o[u]);
+    if constexpr (!kLast) {
+      __builtin_amdgcn_sched_barrier(0);
+      static_for<NS>([&](auto qc) {
+        constexpr int q = qc.value;
+        s_mfma(qc, xn);
+        if constexpr (q + kAhead < 2 * KC) read_k(std::integral_constant<int, q + kAhead>{});
+        else read_v(std::integral_constant<int, q + kAhead - 2 * KC>{});
+        // the probabilities of the first half's keys behind the first half's products (their
+        // scores' registers are then free for the second half's), half of the others' behind the
+        // second half's; the loads of K(b + 2), V(b + 1)
+        static_for<p_of(q + 1, NS) - p_of(q, NS)>([&](auto i) {
+          p_step(std::integral_constant<int, p_of(q, NS) + i.value>{}, x);
+        });
+        if constexpr (q % 4 == 3 && q / 4 < NI)
+          kd.template issue<q / 4 < NI ? q / 4 : 0>(ksrc, k_lds(cur), wave);
+        if constexpr (q % 4 == 1 && q / 4 < NI)
+          vd.template issue<q / 4 < NI ? q / 4 : 0>(vsrc, v_lds(next), wave);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      kd.step(blk_b);
+      vd.step(blk_b);
+    } else {
+      static_for<12>([&](auto i) { p_step(i, x); });
+    }
+    // P V: behind the first half of its products the rest of the probabilities, behind the second
+    // the next block's maximum
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<NV>([&](auto qc) {
+      constexpr int q = qc.value, kk = q / DT, u = q % DT, half = NV / 2;
+      o[u] = mfma(vf[q], pb[kk], o[u]);
+      if constexpr (q + kAhead < NV) read_v(std::integral_constant<int, q + kAhead>{});
+      if constexpr (q < half) {
+        static_for<(q + 1) * 4 / half - q * 4 / half>([&](auto i) {
+          p_step(std::integral_constant<int, 12 + q * 4 / half + i.value>{}, x);
+        });
+      } else if constexpr (!kLast) {
+        if constexpr (q == half) {
+          // max3 is assembly, whose operands the compiler does not wait for: read no earlier than
+          // here, half of P V after the last product of S
+          asm volatile("" : "+v"(xn[0]), "+v"(xn[1]));
+          if constexpr (masked.value) mask(xn, (b + 1) * kKB);
+        }
+        static_for<(q + 1 - half) * 16 / half - (q - half) * 16 / half>([&](auto i) {
+          max_step(std::integral_constant<int, (q - half) * 16 / half + i.value>{}, xn);
+        });
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    if constexpr (!kLast) {
+      mx = pair_max(mx);
+      cur = next;
     }
   };
 
-  for (int kb = kb0; kb < kb1; ++kb) {
-    __syncthreads();
-    sk.store(ks, tid);
-    sv.store(vs, tid);
-    __syncthreads();
-    // the next block (past the sequence: zeros, not used)
-    sk.load(ksrc, (kb + 1) * kKB, kvs_b, tid);
-    sv.load(vsrc, (kb + 1) * kKB, kvs_b, tid);
-    block(kb * kKB);
+  // the first block's scores and maximum
+  sync_tile<2 * NI>();  // K(kb0) landed
+  static_for<2 * KC>([&](auto i) { read_k(i); });
+  static_for<2 * KC>([&](auto q) { s_mfma(q, s); });
+  // max3 is assembly: the products' latency is waited for here
+  asm volatile("s_nop 15\n\ts_nop 15" : "+v"(s[0]), "+v"(s[1]));
+  mask(s, kb0 * kKB);
+  static_for<16>([&](auto i) { max_step(i, s); });
+  mx = pair_max(mx);
+  m = mx * c;
+  // masked from the first block that reaches past the first query on
+  int b = kb0;
+  const int edge = min(q0 / kKB, kb1 - 1);
+  const std::false_type no;
+  const std::true_type yes;
+  for (; b + 2 < edge; b += 2) {  // in pairs: no score changes its registers
+    block(no, no, b, s, sn);
+    block(no, no, b + 1, sn, s);
   }
+  for (; b + 1 < kb1; ++b) {
+    block(no, yes, b, s, sn);
+    s[0] = sn[0];
+    s[1] = sn[1];
+  }
+  block(yes, no, b, s, sn);
+  __builtin_amdgcn_s_waitcnt(0);  // loads past the range: none in flight when the wavefront ends
   const float ltot = lsum + __shfl_xor(lsum, 32, 64);
+  if (!live || qi >= L) return;
   if (nch == 1) {
-    if (qi < L) {
-      store_token_row<D>(a.out + (int64_t)(start + qi) * qs + h * D, o, 1.0f / ltot, lane);
-      if (lane < 32) a.lse[(int64_t)h * a.n + start + qi] = (m + log2f(ltot)) * kLn2;
-    }
+    store_token_row<D>(a.out + (int64_t)(start + qi) * qs + h * D, o, 1.0f / ltot, lane);
+    if (lane < 32) a.lse[(int64_t)h * a.n + start + qi] = (m + log2f(ltot)) * kLn2;
     return;
   }
-  // Several chunks: this one's unnormalised partial and (m, l). Every chunk holds at least one
-  // unmasked key of each query (the last one starts at or before the tile's first query: q0 is
-  // a multiple of 32, blocks are 64 keys; the others precede it), so m is finite.
-  if (qi < L) {
-    store_token_row_f32<D>(a.part + (((int64_t)ch * a.n + start + qi) * a.HQ + h) * D, o, lane);
-    if (lane < 32)
-      a.part_ml[((int64_t)ch * a.HQ + h) * a.n + start + qi] = make_float2(m, ltot);
-  }
+  // Several chunks: this one's unnormalised partial and (m, l). Every chunk of a tile holds at
+  // least one unmasked key of each query (the last one starts at or before the tile's first query:
+  // q0 is a multiple of 32, blocks are 64 keys; the others precede it), so m is finite.
+  store_token_row_f32<D>(a.part + (((int64_t)ch * a.n + start + qi) * a.HQ + h) * D, o, lane);
+  if (lane < 32) a.part_ml[((int64_t)ch * a.HQ + h) * a.n + start + qi] = make_float2(m, ltot);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -718,14 +942,13 @@ int check_common(int32_t nseq, int32_t max_len, int64_t n, int32_t HQ, int32_t K
   return 0;
 }
 
-// MODE: 0 forward, 1 dQ reading delta, 2 dQ forming delta
+// MODE: 1 dQ reading delta, 2 dQ forming delta
 template <int D, int G, int MODE>
 void launch_q(const Args& a, dim3 grid, hipStream_t s) {
   if constexpr (MODE == 1)
     hipLaunchKernelGGL((attn_dq_kernel<D, G, false>), grid, dim3(64 * G), 0, s, a);
-  else if constexpr (MODE == 2)
+  else
     hipLaunchKernelGGL((attn_dq_kernel<D, G, true>), grid, dim3(64 * G), 0, s, a);
-  else hipLaunchKernelGGL((attn_fwd_kernel<D, G>), grid, dim3(64 * G), 0, s, a);
 }
 
 template <int MODE, int D>
@@ -786,13 +1009,30 @@ int launch_merge(const Args& a, int D, int64_t nseq, int64_t nch, hipStream_t s)
   return qlora_launch_status();
 }
 
-int run_fwd(Args a, int32_t nseq, int32_t max_len, int D, int64_t nch, hipStream_t s) {
-  a.ntiles = (int)qlora_cdiv(max_len, kTok);
+template <int D, int NW>
+int launch_fwd(Args a, int32_t nseq, int64_t tiles, int64_t nch, hipStream_t s) {
+  a.ntiles = (int)qlora_cdiv(tiles * (a.HQ / a.KH), NW);
   unsigned gx;
   if (int rc = grid_of(a.ntiles, (int64_t)nseq * a.KH, &gx)) return rc;
-  launch_q_any<0>(a, D, a.HQ / a.KH, dim3(gx, 1, (unsigned)nch), s);
-  if (int rc = qlora_launch_status()) return rc;
-  return nch > 1 ? launch_merge<true>(a, D, nseq, nch, s) : 0;
+  hipLaunchKernelGGL((attn_fwd_kernel<D, NW>), dim3(gx, 1, (unsigned)nch), dim3(64 * NW), 0, s, a);
+  return qlora_launch_status();
+}
+
+// Whether the (query or key tile, head) pairs fill the GPU with workgroups of eight wavefronts.
+bool wide_groups(const Args& a) { return qlora_cdiv(a.n, kTok) * a.HQ >= 2048; }
+
+int run_fwd(Args a, int32_t nseq, int32_t max_len, int D, int64_t nch, hipStream_t s) {
+  const int64_t tiles = qlora_cdiv(max_len, kTok);
+  int rc;
+  if (D == 128)
+    rc = wide_groups(a) ? launch_fwd<128, 8>(a, nseq, tiles, nch, s)
+                        : launch_fwd<128, 4>(a, nseq, tiles, nch, s);
+  else
+    rc = wide_groups(a) ? launch_fwd<64, 8>(a, nseq, tiles, nch, s)
+                        : launch_fwd<64, 4>(a, nseq, tiles, nch, s);
+  a.ntiles = (int)tiles;
+  if (rc == 0 && nch > 1) rc = launch_merge<true>(a, D, nseq, nch, s);
+  return rc;
 }
 
 // The second stream of each device on which the dK/dV kernel runs while the dQ kernel runs on

@@ -5,6 +5,8 @@
 #include <hip/hip_fp16.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #define QLORA_API extern "C" __attribute__((visibility("default")))
 
 // Error convention of every entry point: 0 on success, a hipError_t otherwise. Arguments that a
@@ -82,6 +84,35 @@ __device__ __forceinline__ float buf_load_f32(rsrc_t r, uint32_t off) {
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void buf_store16(rsrc_t r, uint32_t off, uint4 v) {
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), r, off, 0, 0);
+}
+
+// ---- LDS DMA ---------------------------------------------------------------------------------------
+// One DMA instruction (16 bytes a lane) to LDS byte lds (wave-uniform) + 1024 J + 16 lane. The
+// caller waits for it (sync_tile).
+template <int J>
+__device__ __forceinline__ void dma16(rsrc_t r, uint32_t voff, uint32_t lds) {
+  asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds"
+               :
+               : "s"(lds), "n"(1024 * J), "v"(voff), "s"(r)
+               : "scc");
+}
+
+// s_waitcnt with vmcnt(VM) and lgkmcnt(0), then s_barrier: this thread's LDS stores and all
+// but its VM most recent vector-memory loads are done, and so are every other thread's.
+template <int VM>
+__device__ __forceinline__ void sync_tile() {
+  static_assert(VM >= 0 && VM < 64, "vmcnt is 6 bits");
+  __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | (7 << 4));
+  __builtin_amdgcn_s_barrier();
+}
+
+// f(0), f(1), .. f(N - 1), each index a compile-time constant.
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void static_for(F f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(f);
+  }
 }
 
 }  // namespace qlora

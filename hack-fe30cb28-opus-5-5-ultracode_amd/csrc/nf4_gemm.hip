@@ -422,15 +422,6 @@ __device__ __forceinline__ void nf4_decode_part(const uint4& v, float sc, NF4Pla
   }
 }
 
-// s_waitcnt with vmcnt(VM) and lgkmcnt(0), then s_barrier: this thread's LDS stores and all
-// but its VM most recent vector-memory loads are done, and so are every other thread's.
-template <int VM>
-__device__ __forceinline__ void sync_tile() {
-  static_assert(VM >= 0 && VM < 64, "vmcnt is 6 bits");
-  __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | (7 << 4));
-  __builtin_amdgcn_s_barrier();
-}
-
 // Epilogue 5 of a BM x BN tile (registers and LDS areas as store_tile): the product [g | u]
 // first, staged as a plain store would and written to gate column n and up column I + n of g.gu;
 // while those stores issue (they stall when every CU of a round writes at once), the SwiGLU of
@@ -1207,16 +1198,6 @@ constexpr uint32_t kLds256 = 5 * kStageBytes;
 
 typedef __attribute__((address_space(3))) const half8_t lds_half8_t;
 
-// One DMA instruction (16 bytes a lane) to LDS byte lds (wave-uniform) + 1024 J + 16 lane. The
-// caller waits for it (sync_tile).
-template <int J>
-__device__ __forceinline__ void dma16(rsrc_t r, uint32_t voff, uint32_t lds) {
-  asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds"
-               :
-               : "s"(lds), "n"(1024 * J), "v"(voff), "s"(r)
-               : "scc");
-}
-
 // acc += a b in place: in assembly, since with all 256 accumulation registers taken the compiler
 // gives some products another destination and copies them back (NN and transposed A). It then
 // does not see the product's latency either: settle() before anything else reads acc. (In the
@@ -1230,15 +1211,6 @@ __device__ __forceinline__ void settle(Acc16& acc) {
     asm volatile("s_nop 15"
                  : "+a"(acc.a[i][0]), "+a"(acc.a[i][1]), "+a"(acc.a[i][2]), "+a"(acc.a[i][3]),
                    "+a"(acc.a[i][4]), "+a"(acc.a[i][5]), "+a"(acc.a[i][6]), "+a"(acc.a[i][7]));
-}
-
-// f(0), f(1), .. f(N - 1), each index a compile-time constant.
-template <int N, int I = 0, typename F>
-__device__ __forceinline__ void static_for(F f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<N, I + 1>(f);
-  }
 }
 
 // [64][256] (N-contiguous): chunk c of row k in slot c ^ ((k & 3) << 2) ^ ((k >> 3) & 1) << 1. A

@@ -168,3 +168,34 @@ def test_concurrent_backward_other_shapes(pkg, HQ, KH, D):
     own kernel) at other head sizes and group counts (Qwen2 0.5B 14/2 x 64, 3B 16/2, 7B 28/4,
     and one q head per kv head) against fp32 SDPA, key ranges unsplit."""
     _run(pkg, [600, 300], HQ, KH, D, seed=HQ + D, chunk=0)
+
+
+@pytest.mark.parametrize("HQ,KH,D,lengths", [(12, 2, 128, [700, 33]), (14, 2, 64, [700, 33]),
+                                             (12, 2, 128, [1500, 1200, 1100, 1000, 900])])
+def test_forward_rescales_as_scores_grow(pkg, HQ, KH, D, lengths):
+    """Scores that grow along the keys by far more than 2^8 move the forward's reference maximum
+    (and rescale O) in block after block; four and eight wavefronts a workgroup (2,048 tiles and
+    more). Against fp32 SDPA on the GPU; out is a convex combination of v (|v| <= 1 here), p and
+    out are rounded to fp16 once each: 2 x 2^-11 of it."""
+    g = torch.Generator(device=DEV).manual_seed(5)
+    n = sum(lengths)
+    q = torch.rand(n, HQ, D, device=DEV, generator=g).half()
+    v = (torch.rand(n, KH, D, device=DEV, generator=g) * 2 - 1).half()
+    grow = torch.cat([torch.linspace(0, 8, x, device=DEV) for x in lengths])
+    k = (torch.rand(n, KH, D, device=DEV, generator=g) * grow[:, None, None]).half()
+    packed = _Packed(lengths)
+    print(f"attn growing scores lengths={lengths} HQ={HQ} D={D}", flush=True)
+    out, lse, _, _ = pkg.ops._attn_fwd(q, k, v, packed, D ** -0.5)
+    torch.cuda.synchronize()
+    start = 0
+    for x in lengths:
+        sl = slice(start, start + x)
+        qf, kf, vf = (t[sl].float().transpose(0, 1) for t in (q, _expand(k, HQ // KH),
+                                                              _expand(v, HQ // KH)))
+        s = torch.bmm(qf, kf.transpose(1, 2).contiguous()) * D ** -0.5
+        s = s.masked_fill(torch.ones(x, x, device=DEV, dtype=torch.bool).triu(1), float("-inf"))
+        assert s.amax() - s[:, -1, 0].amin() > 12  # several rescales (8 in log2 units each)
+        ref = torch.bmm(torch.softmax(s, -1), vf).transpose(0, 1)
+        assert (out[sl].float() - ref).abs().amax() < 2 * 2 ** -11
+        torch.testing.assert_close(lse[:, sl], torch.logsumexp(s, -1), rtol=1e-5, atol=1e-4)
+        start += x
