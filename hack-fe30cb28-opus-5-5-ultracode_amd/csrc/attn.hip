@@ -17,20 +17,18 @@
 //  * dK/dV compute S = Q K^T (lane <-> key), dV^T = dO^T P and dK^T = Q^T dS.
 // A product that contracts over tokens needs a token-contiguous operand (V^T forward, K^T dQ,
 // Q^T and dO^T dK/dV): the tiles are staged row-major with 16-byte stores and read transposed
-// with ds_read_b64_tr_b16 (tr_operand). The P/dS operand comes straight from the accumulator
+// with ds_read_b64_tr_b16 (TrFrags). The P/dS operand comes straight from the accumulator
 // registers, whose rows within each 16-row group are in the order 0-3, 8-11, 4-7, 12-15 for the
-// lower/upper half-wave; tr_operand hands out the tokens in that same order, so no register
+// lower/upper half-wave; TrFrags hands out the tokens in that same order, so no register
 // shuffles are needed.
 // LDS tiles are XOR-swizzled by 16-byte chunk so that the operand reads (32 rows, same chunk)
 // and the staging writes are spread over the banks.
 //
-// One workgroup = consecutive (query tile, q head) pairs of one kv head (forward) or the q heads
-// that share a kv head (dQ), which share the staged K/V tiles; dK/dV: four wavefronts on 128
-// consecutive keys of one q head, sharing the staged Q/dO. The next tile's loads are in flight
-// during the current tile's MFMAs (forward: LDS DMA; dQ, dK/dV: global loads into registers, a
-// prefetch), so their latency overlaps the arithmetic. dK/dV come out per q head
-// ([n, HQ, D]); the caller sums each group (the RoPE backward does, as the reference sums the
-// repeated kv heads). The log-sum-exp of the forward (natural log, fp32 [HQ, n]) and
+// One workgroup = consecutive (query tile, q head) pairs of one kv head (forward, dQ), which share
+// the staged K/V tiles; dK/dV: four wavefronts on 128 consecutive keys of one q head, sharing the
+// staged Q/dO. The next tiles arrive by LDS DMA during the current tile's MFMAs. dK/dV come out
+// per q head ([n, HQ, D]); the caller sums each group (the RoPE backward does, as the reference
+// sums the repeated kv heads). The log-sum-exp of the forward (natural log, fp32 [HQ, n]) and
 // delta = rowsum(dO * O) (fp32 [HQ, n], written by attn_delta_kernel) feed the dQ and the dK/dV
 // kernels, which run at the same time on two streams.
 #include "common.h"
@@ -92,7 +90,7 @@ __host__ __device__ constexpr int rm_off(int row, int chunk) {
   return row * D + ((chunk ^ (row & (D / 8 - 1))) << 3);
 }
 
-// [rows][D] tile read transposed by ds_read_b64_tr_b16 (tr_operand): a half-wave reads 4
+// [rows][D] tile read transposed by ds_read_b64_tr_b16 (TrFrags): a half-wave reads 4
 // consecutive rows (the first a multiple of 4) x 4 aligned chunks, which this swizzle spreads
 // over distinct banks; 16-byte row stores (16 threads a row) stay conflict-free too.
 template <int D>
@@ -104,71 +102,6 @@ __host__ __device__ constexpr int tt_off(int row, int chunk) {
 
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) short4_t lds_short4_t;
-
-// The MFMA A operand T[d][8 token slots] of a tt_off tile (T = the tile transposed): lane l
-// supplies d = d0 + l % 32 and tokens k0 + 4 (l / 32) + {0..3, 8..11}, the slot order of an
-// accumulator's rows (acc_row). ds_read_b64_tr_b16 gives lane i of each 16-lane group element
-// i % 4 of the 4 halves read by lane 4 j + i / 4 of the group, as its element j; so lane p of the
-// group reads row (first token) + p / 4, columns (group's first d) + 4 (p % 4) .. + 3.
-template <int D>
-__device__ __forceinline__ half8_t tr_operand(const uint16_t* t, int k0, int d0, int lane) {
-  const int p = lane & 15;
-  const int row = k0 + 4 * (lane >> 5) + (p >> 2);
-  const int col = d0 + 16 * ((lane >> 4) & 1) + 4 * (p & 3);
-  const int o0 = tt_off<D>(row, col >> 3) + (col & 7);
-  const int o1 = tt_off<D>(row + 8, col >> 3) + (col & 7);
-  const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(t + o0));
-  const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(t + o1));
-  return __builtin_bit_cast(half8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-}
-
-// A row operand (as ld_rm) of a tt_off tile: the swizzle maps 16 consecutive rows of one chunk
-// to distinct banks too.
-template <int D>
-__device__ __forceinline__ half8_t ld_tt(const uint16_t* t, int row, int chunk) {
-  return *reinterpret_cast<const half8_t*>(t + tt_off<D>(row, chunk));
-}
-
-template <int D>
-__device__ __forceinline__ half8_t ld_rm(const uint16_t* t, int row, int chunk) {
-  return *reinterpret_cast<const half8_t*>(t + rm_off<D>(row, chunk));
-}
-__device__ __forceinline__ half8_t ld_g(const uint16_t* p) {
-  return *reinterpret_cast<const half8_t*>(p);
-}
-
-// Staging of token-major global rows into LDS tiles, split into a load phase (all of a thread's
-// global loads issued back to back into registers, so their latencies overlap, and early enough
-// to hide behind the previous tile's MFMAs) and a store phase into the tile. The loads are
-// buffer loads over the sequence's rows of one head: rows past the sequence read zeros, so
-// there is neither a clamp nor a select on the loaded value (which the compiler may turn into a
-// branch around the load, whose join then waits for every load in flight).
-//
-// Offsets are bytes from the resource base: row r at r * stride_b, chunk c (8 halves) at 16 c.
-//
-// RowStage: rows [row0, row0 + ROWS) into a [ROWS][D] tile (swizzle rm_off, or tt_off for a
-// tile read by tr_operand).
-template <int D, int ROWS, int NT, bool TT = false>
-struct RowStage {
-  static constexpr int CPR = D / 8, TOTAL = ROWS * CPR, CNT = (TOTAL + NT - 1) / NT;
-  uint4 r[CNT];
-  __device__ __forceinline__ void load(rsrc_t src, int row0, int stride_b, int tid) {
-#pragma unroll
-    for (int i = 0; i < CNT; ++i) {
-      const int id = tid + i * NT, row = id / CPR, c = id % CPR;  // id >= TOTAL: not stored
-      r[i] = buf_load16(src, (uint32_t)((row0 + row) * stride_b + c * 16));
-    }
-  }
-  __device__ __forceinline__ void store(uint16_t* tile, int tid) const {
-#pragma unroll
-    for (int i = 0; i < CNT; ++i) {
-      const int id = tid + i * NT;
-      if (id < TOTAL)
-        *reinterpret_cast<uint4*>(tile + (TT ? tt_off<D>(id / CPR, id % CPR)
-                                             : rm_off<D>(id / CPR, id % CPR))) = r[i];
-    }
-  }
-};
 
 __device__ __forceinline__ uint32_t word_of(const uint4& x, int i) {
   return i < 2 ? (i == 0 ? x.x : x.y) : (i == 2 ? x.z : x.w);
@@ -188,14 +121,6 @@ __device__ __forceinline__ void load_token(rsrc_t src, int row, int stride_b, in
   for (int kk = 0; kk < D / 16; ++kk)
     out[kk] = __builtin_bit_cast(
         half8_t, buf_load16(src, (uint32_t)(row * stride_b + (2 * kk + (lane >> 5)) * 16)));
-}
-
-// 8 accumulator values (registers 8 * half .. + 7 of acc) as an fp16 B operand.
-__device__ __forceinline__ half8_t to_b(const f32x16& acc, int half) {
-  half8_t r;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) r[i] = (_Float16)acc[8 * half + i];
-  return r;
 }
 
 // Row (query or key) index within the 32 x 32 tile of register r for this lane.
@@ -281,7 +206,8 @@ template <int D, bool TT = false>
 struct RowFrags {
   uint32_t at[D / 16];
   __device__ __forceinline__ void set(uint32_t stage, int lane) {
-    const uint32_t l0 = (uint32_t)(2 * (TT ? tt_off<D>(lane & 31, lane >> 5) : rm_off<D>(lane & 31, lane >> 5)));
+    const int row = lane & 31, chunk = lane >> 5;
+    const uint32_t l0 = (uint32_t)(2 * (TT ? tt_off<D>(row, chunk) : rm_off<D>(row, chunk)));
 #pragma unroll
     for (int kk = 0; kk < D / 16; ++kk) at[kk] = l0 ^ (uint32_t)(32 * kk);
     move(stage);
@@ -297,7 +223,12 @@ struct RowFrags {
     return *(lds_half8_t*)(uintptr_t)(at[kk] + (uint32_t)(half * 32 * D * 2));
   }
 };
-// tt_off stage read transposed: fragment (kk, u): tokens 16 kk .., columns 32 u .. (tr_operand).
+// tt_off stage read transposed: fragment (kk, u) is the A operand T[d][8 token slots] (T = the
+// stage transposed) of tokens k0 = 16 kk .., columns d0 = 32 u ..
+// Lane l supplies d = d0 + l % 32 and tokens k0 + 4 (l / 32) + {0..3, 8..11}, the slot order of an
+// accumulator's rows (acc_row). ds_read_b64_tr_b16 gives lane i of each 16-lane group element
+// i % 4 of the 4 halves read by lane 4 j + i / 4 of the group, as its element j; so lane p of the
+// group reads row (first token) + p / 4, columns (group's first d) + 4 (p % 4) .. + 3.
 template <int D>
 struct TrFrags {
   uint32_t lo[D / 32], hi[D / 32];
@@ -321,7 +252,8 @@ struct TrFrags {
     }
   }
   __device__ __forceinline__ half8_t get(int kk, int u) const {
-    const uint32_t a0 = lo[u] + (uint32_t)(16 * kk * D * 2), a1 = hi[u] + (uint32_t)((16 * kk + 8) * D * 2);
+    const uint32_t a0 = lo[u] + (uint32_t)(16 * kk * D * 2);
+    const uint32_t a1 = hi[u] + (uint32_t)((16 * kk + 8) * D * 2);
     const short4_t x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(uintptr_t)a0);
     const short4_t y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(uintptr_t)a1);
     return __builtin_bit_cast(half8_t, __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7));
@@ -628,40 +560,97 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(const uint16_t* dout, c
 }
 
 // ------------------------------------------------------------------------------------------------
-// Backward, dQ: per 32 queries of a q head, over 32-key blocks up to the diagonal: S^T = K Q^T,
-// P = exp(S - lse), dP^T = V dO^T, dS = P (dP - delta), dQ^T += K^T dS^T. grid and block as the
-// forward; block kb + 1 prefetched during block kb. OWN_DELTA: the kernel forms delta itself
-// (lanes l and l ^ 32 sum the chunks of attn_delta_kernel's two threads, in its order) and the
-// first chunk writes it for the dK/dV kernel that follows; else it reads attn_delta_kernel's.
+// Staging of the backward kernels: blocks of 32 rows of two token-major matrices with the same
+// rows and stride (K and V for dQ, Q and dO for dK/dV), as one [64][D] tt_off stage of LDS: rows
+// 0-31 the first matrix, 32-63 the second, so that one set of fragment addresses reaches both
+// (RowFrags: (kk, matrix), TrFrags: (kk + 2 matrix, u)).
 // ------------------------------------------------------------------------------------------------
-template <int D, int G, bool OWN_DELTA>
-__global__ __launch_bounds__(64 * G) void attn_dq_kernel(Args a) {
-  constexpr int KC = D / 16, DT = D / 32, NT = 64 * G, KB = kTok;
-  __shared__ __align__(16) uint16_t ks[KB * D];  // tt_off: read by rows and transposed
-  __shared__ __align__(16) uint16_t vs[KB * D];
-  const int sh = blockIdx.x / a.ntiles;  // as the forward
-  const int tile = a.ntiles - 1 - (int)(blockIdx.x - sh * a.ntiles);
+template <int D, int NW>
+struct PairDma {
+  typedef BlockDma<D, kTok, NW, true> Dma;
+  static constexpr int N = 2 * Dma::N;           // instructions a wavefront and block
+  static constexpr uint32_t kHalf = kTok * D * 2, kStage = 2 * kHalf;  // bytes
+  Dma d;
+  __device__ __forceinline__ void init(int row0, int stride_b, int lane, int wave) {
+    d.init(row0, stride_b, lane, wave);
+  }
+  template <int J>
+  __device__ __forceinline__ void issue(rsrc_t first, rsrc_t second, uint32_t stage,
+                                        int wave) const {
+    if constexpr (J < Dma::N) d.template issue<J>(first, stage, wave);
+    else d.template issue<J - Dma::N>(second, stage + kHalf, wave);
+  }
+};
+
+// Halves 2 i and 2 i + 1 of a fragment.
+__device__ __forceinline__ void set_pair(half8_t& f, int i, uint32_t pair) {
+  uint4 w = __builtin_bit_cast(uint4, f);
+  (i == 0 ? w.x : i == 1 ? w.y : i == 2 ? w.z : w.w) = pair;
+  f = __builtin_bit_cast(half8_t, w);
+}
+
+// Steps of a block's dS (of 8) formed before MFMA q of the 3 D / 16 they hide behind: the second
+// half of the dQ products of the block before, the next block's S and dP, the first half of its own
+// dQ.
+template <int D>
+constexpr int ds_before(int q) {
+  return q * 8 / (3 * D / 16);
+}
+
+// ------------------------------------------------------------------------------------------------
+// Backward, dQ: per 32 queries of a q head, over 32-key blocks up to the diagonal: S^T = K Q^T,
+// P = exp(S - lse), dP^T = V dO^T, dS = P (dP - delta), dQ^T += K^T dS^T. Workgroups, their order
+// and the chunks as the forward. Block b's dS is formed a few instructions at a time (ds_step)
+// behind the MFMAs of block b + 1's S and dP and of block b's dQ, as in attn_dkdv_kernel; K and V
+// arrive by LDS DMA, four stages, one barrier a block, and masks start at the diagonal.
+// MI355X, 12/2 heads of 128, against one q head group per workgroup, staging through registers and
+// two barriers a block: sequences of 4,096 and 3,001 tokens 200 -> 143 us, four of 283-997 44 -> 34.
+// OWN_DELTA: the kernel forms delta itself (lanes l and l ^ 32 sum the chunks of
+// attn_delta_kernel's two threads, in its order) and the first chunk writes it for the dK/dV
+// kernel that follows; else it reads attn_delta_kernel's.
+// ------------------------------------------------------------------------------------------------
+template <int D, int NW, bool OWN_DELTA>
+__global__ __launch_bounds__(64 * NW, 2) void attn_dq_kernel(Args a) {
+  constexpr int KC = D / 16, DT = D / 32, kStages = 4;
+  typedef PairDma<D, NW> Dma;
+  constexpr int NL = Dma::N;  // loads a wavefront and block
+  __shared__ __align__(1024) uint8_t smem[kStages * Dma::kStage];
+  const int G = a.HQ / a.KH;
+  const int pairs = gridDim.x / a.ntiles, rank = blockIdx.x / pairs;  // as the forward
+  const int sh = ((int)blockIdx.x - rank * pairs + rank) % pairs, grp = a.ntiles - 1 - rank;
   const int seq = sh / a.KH, kvh = sh % a.KH;
-  const int q0 = tile * kTok;
   const int start = a.cu[seq], L = a.cu[seq + 1] - start;
-  if (q0 >= L) return;
+  const int total = (L + kTok - 1) / kTok * G;
+  if (grp * NW >= total) return;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int h = kvh * G + __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
-  const int qi = q0 + (lane & 31);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  auto blocks_of = [&](int f) { return f / G + 1; };  // key blocks are as long as query tiles
+  const int nkb = blocks_of(min(grp * NW + NW - 1, total - 1));  // of the longest tile
+  const int ch = blockIdx.z;
+  if (ch >= num_chunks(nkb, a.chunk)) return;
+  const int kb0 = ch * a.chunk, kb1 = num_chunks(nkb, a.chunk) == 1 ? nkb : min(nkb, kb0 + a.chunk);
+
   const int64_t qs = (int64_t)a.HQ * D, kvs = (int64_t)a.KH * D;
   const int qs_b = (int)(qs * 2), kvs_b = (int)(kvs * 2);
-  const int kend = min(q0 + kTok, L);
-  const int nkb = (kend + KB - 1) / KB;
-  const int nch = num_chunks(nkb, a.chunk), ch = blockIdx.z;
-  if (ch >= nch) return;
-  const int kb0 = ch * a.chunk, kb1 = nch == 1 ? nkb : min(nkb, kb0 + a.chunk);
   const rsrc_t ksrc = rows_rsrc(a.k + (int64_t)start * kvs + kvh * D, L, kvs, D);
   const rsrc_t vsrc = rows_rsrc(a.v + (int64_t)start * kvs + kvh * D, L, kvs, D);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
+  Dma dma;
+  dma.init(kb0 * kTok, kvs_b, lane, wave);
+  auto stage_at = [&](int b) { return lds0 + (uint32_t)(b & (kStages - 1)) * Dma::kStage; };
+  auto load = [&](auto j, int b) {  // load j of block b; the last moves to the next block
+    dma.template issue<j.value>(ksrc, vsrc, stage_at(b), wave);
+    if constexpr (j.value == NL - 1) dma.d.step((uint32_t)(kTok * kvs_b));
+  };
+  for (int b = kb0; b < kb0 + 3; ++b) static_for<NL>([&](auto j) { load(j, b); });
 
-  RowStage<D, KB, NT, true> sk;  // K: one tile for S^T = K Q^T and K^T (tr_operand)
-  RowStage<D, KB, NT> sv;
-  sk.load(ksrc, kb0 * KB, kvs_b, tid);
-  sv.load(vsrc, kb0 * KB, kvs_b, tid);
+  // the wavefront's tile, as the forward: past the last tile the last one again, not stored
+  const int f = grp * NW + wave, fc = min(f, total - 1);
+  const int h = kvh * G + __builtin_amdgcn_readfirstlane(fc % G);
+  const int q0 = __builtin_amdgcn_readfirstlane(fc / G) * kTok;
+  const int qi = q0 + (lane & 31), lim = min(qi, L - 1);
+  const int nch = num_chunks(blocks_of(fc), a.chunk);
+  const bool live = f < total && ch < nch;
 
   // this query's q and dO (queries past the sequence read zeros; their dq is not stored), its
   // log-sum-exp and delta (attn_delta_kernel)
@@ -682,59 +671,126 @@ __global__ __launch_bounds__(64 * G) void attn_dq_kernel(Args a) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) dpart += (float)dr[kk][i] * (float)orow[kk][i];
     delta = dpart + __shfl_xor(dpart, 32, 64);
-    if (ch == 0 && qi < L && lane < 32) a.delta[(int64_t)h * a.n + start + qi] = delta;
+    if (live && ch == 0 && qi < L && lane < 32) a.delta[(int64_t)h * a.n + start + qi] = delta;
   } else {
     delta = buf_load_f32(make_rsrc(a.delta + (int64_t)h * a.n + start, (uint32_t)L * 4), qi * 4);
   }
 
-  f32x16 dq[DT];
+  f32x16 dq[DT], s[2], sn[2];  // s: S and dP
 #pragma unroll
   for (int u = 0; u < DT; ++u) dq[u] = f32x16{};
   const float c = a.scale * kLog2e;
-  const int lim = min(qi, L - 1);
+  half8_t sb[2];  // dS fragments
+  RowFrags<D, true> rat;
+  TrFrags<D> tat;
+  uint32_t r_at = stage_at(kb0), t_at = r_at;  // the stages rat and tat address
+  rat.set(r_at, lane);
+  tat.set(t_at, lane);
+  half8_t rf[2 * KC], tf[2 * DT];
+  // MFMA q of S, dP: row fragment q (even: K, odd: V); of dQ: transposed fragment q (first the
+  // first 16 keys)
+  auto read_r = [&](auto i) { rf[i.value] = rat.get(i.value >> 1, i.value & 1); };
+  auto read_t = [&](auto i) { tf[i.value] = tat.get(i.value / DT, i.value % DT); };
+  auto s_mfma = [&](auto qc, f32x16 (&x)[2]) {
+    constexpr int kk = qc.value >> 1, t = qc.value & 1;
+    x[t] = mfma(rf[qc.value], t ? dr[kk] : qr[kk], kk == 0 ? f32x16{} : x[t]);
+  };
+  // dS of keys acc_row(2 k) and the next (k = 0 .. 7)
+  auto ds_step = [&](auto kc, f32x16 (&x)[2]) {
+    constexpr int r = 2 * kc.value;
+    const float p0 = ex2(fmaf(x[0][r], c, -lse2)), p1 = ex2(fmaf(x[0][r + 1], c, -lse2));
+    set_pair(sb[r >> 3], (r & 7) >> 1, cvt2h(p0 * (x[1][r] - delta), p1 * (x[1][r + 1] - delta)));
+  };
+  // keys past the query: P = dS = 0
+  auto mask = [&](int b, f32x16 (&x)[2]) {
+    const int d = lim - b * kTok - 4 * (lane >> 5);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) x[0][r] = acc_row(r, 0) > d ? -__builtin_inff() : x[0][r];
+  };
+  constexpr int NS = 2 * KC, NV = 2 * DT, half = NV / 2;  // MFMAs of S and dP, of dQ
+  constexpr int kAhead = 3;  // fragment reads issued ahead of their MFMAs
 
-  for (int kb = kb0; kb < kb1; ++kb) {
-    const int k0 = kb * KB;
-    __syncthreads();
-    sk.store(ks, tid);
-    sv.store(vs, tid);
-    __syncthreads();
-    sk.load(ksrc, k0 + KB, kvs_b, tid);
-    sv.load(vsrc, k0 + KB, kvs_b, tid);
-    f32x16 s = f32x16{}, dp = f32x16{};
-#pragma unroll
-    for (int kk = 0; kk < KC; ++kk) {
-      const int row = lane & 31, ch = 2 * kk + (lane >> 5);
-      const half8_t kop = ld_tt<D>(ks, row, ch), vop = ld_rm<D>(vs, row, ch);
-      s = mfma(kop, qr[kk], s);
-      dp = mfma(vop, dr[kk], dp);
+  // Block b, its S and dP in x and the first steps of its dS done: the next block's go to xn.
+  // last: there is none; masked: it reaches past the first query.
+  auto block = [&](auto last, auto masked, int b, f32x16 (&x)[2], f32x16 (&xn)[2]) {
+    constexpr bool kLast = last.value;
+    sync_tile<NL>();  // block b + 1 landed, every wavefront is done with b - 1
+    if (!kLast) {
+      rat.move(stage_at(b + 1) - r_at);
+      r_at = stage_at(b + 1);
     }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = ex2(fmaf(s[r], c, -lse2));
-    if (k0 + KB - 1 > q0) {  // a block on the diagonal (uniform)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = k0 + acc_row(r, lane) > lim ? 0.f : s[r];
+    tat.move(stage_at(b) - t_at);
+    t_at = stage_at(b);
+    if constexpr (!kLast) {
+      static_for<kAhead>([&](auto i) { read_r(i); });
+      __builtin_amdgcn_sched_barrier(0);
+      static_for<NS>([&](auto qc) {
+        constexpr int q = qc.value, p = ds_before<D>(half + q);
+        s_mfma(qc, xn);
+        if constexpr (q + kAhead < NS) read_r(std::integral_constant<int, q + kAhead>{});
+        else read_t(std::integral_constant<int, q + kAhead - NS>{});
+        static_for<ds_before<D>(half + q + 1) - p>([&](auto i) {
+          ds_step(std::integral_constant<int, p + i.value>{}, x);
+        });
+        if constexpr (q % 3 == 1 && q / 3 < NL) load(std::integral_constant<int, q / 3>{}, b + 3);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    } else {
+      static_for<kAhead>([&](auto i) { read_t(i); });
+      static_for<ds_before<D>(half + NS) - ds_before<D>(half)>([&](auto i) {
+        ds_step(std::integral_constant<int, ds_before<D>(half) + i.value>{}, x);
+      });
+      __builtin_amdgcn_sched_barrier(0);
     }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] *= dp[r] - delta;
-    half8_t sb[2];
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) sb[kk] = to_b(s, kk);
-#pragma unroll
-    for (int u = 0; u < DT; ++u) {
-      const half8_t t0 = tr_operand<D>(ks, 0, 32 * u, lane);
-      const half8_t t1 = tr_operand<D>(ks, 16, 32 * u, lane);
-      dq[u] = mfma(t0, sb[0], dq[u]);
-      dq[u] = mfma(t1, sb[1], dq[u]);
-    }
+    static_for<NV>([&](auto qc) {
+      constexpr int q = qc.value, kk = q / DT, u = q % DT;
+      dq[u] = mfma(tf[q], sb[kk], dq[u]);
+      if constexpr (q + kAhead < NV) read_t(std::integral_constant<int, q + kAhead>{});
+      if constexpr (q < half) {
+        constexpr int p = ds_before<D>(half + NS + q);
+        static_for<ds_before<D>(half + NS + q + 1) - p>([&](auto i) {
+          ds_step(std::integral_constant<int, p + i.value>{}, x);
+        });
+        if constexpr (!kLast && masked.value && q == half - 1) mask(b + 1, xn);
+      } else if constexpr (!kLast) {
+        constexpr int p = ds_before<D>(q - half);
+        static_for<ds_before<D>(q - half + 1) - p>([&](auto i) {
+          ds_step(std::integral_constant<int, p + i.value>{}, xn);
+        });
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  static_assert(3 * (NL - 1) + 1 < NS, "a block's loads are issued behind S and dP");
+  static_assert(ds_before<D>(half + NS) >= 4, "the first 16 keys' dS is whole before dQ");
+
+  sync_tile<2 * NL>();  // the first block landed
+  static_for<NS>([&](auto i) { read_r(i); });
+  static_for<NS>([&](auto q) { s_mfma(q, s); });
+  mask(kb0, s);
+  static_for<ds_before<D>(half)>([&](auto i) { ds_step(i, s); });
+  const std::false_type no;
+  const std::true_type yes;
+  int b = kb0;
+  const int edge = min(q0 / kTok, kb1 - 1);
+  for (; b + 2 < edge; b += 2) {  // in pairs: no product changes its registers
+    block(no, no, b, s, sn);
+    block(no, no, b + 1, sn, s);
   }
+  for (; b + 1 < kb1; ++b) {
+    block(no, yes, b, s, sn);
+    s[0] = sn[0];
+    s[1] = sn[1];
+  }
+  block(yes, no, b, s, sn);
+  __builtin_amdgcn_s_waitcnt(0);  // loads past the range: none in flight when the wavefront ends
+  if (!live || qi >= L) return;
   if (nch == 1) {
-    if (qi < L) store_token_row<D>(a.out + (int64_t)(start + qi) * qs + h * D, dq, a.scale, lane);
+    store_token_row<D>(a.out + (int64_t)(start + qi) * qs + h * D, dq, a.scale, lane);
     return;
   }
   // several chunks: this one's unscaled partial
-  if (qi < L)
-    store_token_row_f32<D>(a.part + (((int64_t)ch * a.n + start + qi) * a.HQ + h) * D, dq, lane);
+  store_token_row_f32<D>(a.part + (((int64_t)ch * a.n + start + qi) * a.HQ + h) * D, dq, lane);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -801,21 +857,29 @@ __global__ __launch_bounds__(32 * D / 4) void attn_merge_kernel(Args a) {
 
 // ------------------------------------------------------------------------------------------------
 // Backward, dK and dV of one q head: a workgroup of 4 wavefronts owns 128 consecutive keys (32
-// per wavefront) and walks the 32-query blocks from its first key to the end of the sequence,
-// staging each block's Q and dO (rows and transposed, plus lse and delta) once for the four
-// wavefronts: S = Q K^T, P = exp(S - lse), dP = dO V^T, dS = P (dP - delta), dV^T += dO^T P,
-// dK^T += Q^T dS. A wavefront skips query blocks that lie wholly before its keys.
+// per wavefront) and walks the 32-query blocks from its first key to the end of the sequence:
+// S = Q K^T, P = exp(S - lse), dP = dO V^T, dS = P (dP - delta), dV^T += dO^T P, dK^T += Q^T dS.
+//
+// dK, dV, K and V take 192 registers a lane (D = 128), so one wavefront runs per SIMD and a block's
+// own products cannot hide its exponentials: block b's P and dS are formed a few instructions at a
+// time (p_sub) behind the MFMAs of block b + 1's S and dP and of block b's dV and dK, every
+// instruction pinned behind an MFMA by sched_barrier. Per block and wavefront 32 MFMAs (D = 128;
+// 1,024 cycles of the matrix core) stand beside about 150 VALU instructions. Q and dO arrive by LDS
+// DMA, four stages (two blocks' time to land), one barrier a block; rows past the sequence read
+// zeros, which add nothing, so only the first four blocks (the diagonal) are masked.
+// MI355X, 12/2 heads of 128, against two barriers a block, staging through registers and a block's
+// products, exponentials and products one after the other: two sequences of 4,096 and 3,001 tokens
+// 290 -> 216 us, four of 283-997 58 -> 43.
 // grid (nseq * HQ * ceil(max_len / 128)), block 256.
 // ------------------------------------------------------------------------------------------------
 constexpr int kKeyWaves = 4;
 
 template <int D>
-__global__ __launch_bounds__(64 * kKeyWaves) void attn_dkdv_kernel(Args a) {
-  constexpr int KC = D / 16, DT = D / 32, NT = 64 * kKeyWaves;
-  __shared__ __align__(16) uint16_t qsm[kTok * D];  // tt_off: read by rows and transposed
-  __shared__ __align__(16) uint16_t dsm[kTok * D];
-  __shared__ __align__(16) float lse_s[kTok];
-  __shared__ __align__(16) float dl_s[kTok];
+__global__ __launch_bounds__(64 * kKeyWaves, 1) void attn_dkdv_kernel(Args a) {
+  constexpr int KC = D / 16, DT = D / 32, kStages = 4;
+  typedef PairDma<D, kKeyWaves> Dma;
+  constexpr uint32_t kRowBytes = kStages * Dma::kStage;  // then per stage lse and delta, 64 floats each
+  __shared__ __align__(1024) uint8_t smem[kRowBytes + kStages * 512];
   // blockIdx.x = (seq HQ + h) + pairs key tile: the first key tiles of every sequence and head,
   // which walk the most queries, are dispatched first (with more workgroups than CUs, the
   // heaviest then do not wait for a free CU)
@@ -828,27 +892,34 @@ __global__ __launch_bounds__(64 * kKeyWaves) void attn_dkdv_kernel(Args a) {
   if (kw0 >= L) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int k0 = kw0 + kTok * wave;
-  const int kj = k0 + (lane & 31);
+  const int kj = kw0 + kTok * wave + (lane & 31);
+  const int nb = (L - kw0 + kTok - 1) / kTok;  // query blocks
   const int64_t qs = (int64_t)a.HQ * D, kvs = (int64_t)a.KH * D;
   const int qs_b = (int)(qs * 2), kvs_b = (int)(kvs * 2);
   const int64_t hoff = (int64_t)start * qs + h * D;
   const rsrc_t qsrc = rows_rsrc(a.q + hoff, L, qs, D);
   const rsrc_t dsrc = rows_rsrc(a.dout + hoff, L, qs, D);
-  const rsrc_t lsrc = make_rsrc(a.lse + (int64_t)h * a.n + start, (uint32_t)L * 4);
-  const rsrc_t dlsrc = make_rsrc(a.delta + (int64_t)h * a.n + start, (uint32_t)L * 4);
+  // even wavefronts fetch a block's lse, odd ones its delta (64 values, the first 32 are used)
+  const rsrc_t rsrc = make_rsrc(((wave & 1) ? a.delta : a.lse) + (int64_t)h * a.n + start,
+                                (uint32_t)L * 4);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
+  const uint32_t row_lds = lds0 + kRowBytes + (uint32_t)(wave & 1) * 256;
 
-  RowStage<D, kTok, NT, true> sq, sd;
-  float lv = 0.f;  // threads 0..31: lse (log2) of query q0 + tid; 32..63: delta of q0 + tid - 32
-  const float first = tid < kTok ? 1.f : 0.f;
-  auto load = [&](int q0) {
-    sq.load(qsrc, q0, qs_b, tid);
-    sd.load(dsrc, q0, qs_b, tid);
-    const uint32_t off = (uint32_t)(q0 + (tid & (kTok - 1))) * 4;
-    const float xl = buf_load_f32(lsrc, off), xd = buf_load_f32(dlsrc, off);
-    lv = fmaf(first, xl * kLog2e, (1.f - first) * xd);  // a blend, not a select of loads
+  Dma dma;
+  dma.init(kw0, qs_b, lane, wave);
+  uint32_t row_off = (uint32_t)(kw0 + lane) * 4;
+  constexpr int NL = Dma::N + 1;  // loads a wavefront and block
+  auto stage_at = [&](int b) { return lds0 + (uint32_t)(b & (kStages - 1)) * Dma::kStage; };
+  auto load = [&](auto j, int b) {  // load j of block b (j = NL - 1, the last, moves to the next)
+    if constexpr (j.value < Dma::N) {
+      dma.template issue<j.value>(qsrc, dsrc, stage_at(b), wave);
+    } else {
+      dma4(rsrc, row_off, row_lds + (uint32_t)(b & (kStages - 1)) * 512);
+      dma.d.step((uint32_t)(kTok * qs_b));
+      row_off += kTok * 4;
+    }
   };
-  load(kw0);
+  for (int b = 0; b < 3; ++b) static_for<NL>([&](auto j) { load(j, b); });
 
   half8_t kr[KC], vr[KC];  // keys past the sequence read zeros (their rows are not stored)
   {
@@ -856,64 +927,157 @@ __global__ __launch_bounds__(64 * kKeyWaves) void attn_dkdv_kernel(Args a) {
     load_token<D>(rows_rsrc(a.k + koff, L, kvs, D), kj, kvs_b, lane, kr);
     load_token<D>(rows_rsrc(a.v + koff, L, kvs, D), kj, kvs_b, lane, vr);
   }
-  f32x16 dk[DT], dv[DT];
+  f32x16 dk[DT], dv[DT], s[2], sn[2];  // s: S and dP
 #pragma unroll
   for (int u = 0; u < DT; ++u) dk[u] = dv[u] = f32x16{};
   const float c = a.scale * kLog2e;
+  half8_t pb[2], sb[2];  // P and dS fragments
+  float4 l4[4], d4[4];   // lse and delta of queries 8 j + 4 (lane / 32) ..
+  RowFrags<D, true> rat;
+  TrFrags<D> tat;
+  rat.set(lds0, lane);
+  tat.set(lds0, lane);
+  uint32_t r_at = lds0, t_at = lds0;  // the stages rat and tat address
+  half8_t rf[2 * KC], tf[4 * DT];
+  // MFMA q of S, dP: row fragment q (even: Q, odd: dO); q of dV, dK: transposed fragment q (first
+  // the first 16 queries; even: dO, odd: Q)
+  auto read_r = [&](auto i) { rf[i.value] = rat.get(i.value >> 1, i.value & 1); };
+  auto read_t = [&](auto i) {
+    constexpr int kk = i.value / (2 * DT), u = i.value % (2 * DT) >> 1;
+    tf[i.value] = tat.get(kk + 2 * (1 - (i.value & 1)), u);
+  };
+  auto s_mfma = [&](auto qc, f32x16 (&x)[2]) {
+    constexpr int kk = qc.value >> 1, t = qc.value & 1;
+    x[t] = mfma(rf[qc.value], t ? vr[kk] : kr[kk], kk == 0 ? f32x16{} : x[t]);
+  };
+  auto g_mfma = [&](auto qc) {
+    constexpr int kk = qc.value / (2 * DT), u = qc.value % (2 * DT) >> 1;
+    if constexpr (qc.value & 1) dk[u] = mfma(tf[qc.value], sb[kk], dk[u]);
+    else dv[u] = mfma(tf[qc.value], pb[kk], dv[u]);
+  };
+  auto move_rows = [&](int b) {
+    rat.move(stage_at(b) - r_at);
+    r_at = stage_at(b);
+  };
+  // the address of block b's lse and delta for this half of the lanes
+  auto row_at = [&](int b) {
+    uint32_t at = lds0 + kRowBytes + (uint32_t)(b & (kStages - 1)) * 512 + 16 * (lane >> 5);
+    asm volatile("" : "+v"(at));  // not read before here
+    return at;
+  };
+  auto read_rows = [&](auto j, uint32_t at) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) const f4 lds_f4_t;
+    l4[j.value] = __builtin_bit_cast(float4, *(lds_f4_t*)(uintptr_t)(at + 32 * j.value));
+    d4[j.value] = __builtin_bit_cast(float4, *(lds_f4_t*)(uintptr_t)(at + 256 + 32 * j.value));
+  };
+  // Part k % 4 of the P and dS of queries acc_row(2 (k / 4)) and the next (k = 0 .. 31)
+  auto p_sub = [&](auto kc, f32x16 (&x)[2]) {
+    constexpr int r = 2 * (kc.value >> 2), part = kc.value & 3;
+    const float4 lj = l4[r >> 2], dj = d4[r >> 2];
+    if constexpr (part == 0) x[0][r] = ex2(fmaf(x[0][r], c, -((r & 2 ? lj.z : lj.x) * kLog2e)));
+    if constexpr (part == 1)
+      x[0][r + 1] = ex2(fmaf(x[0][r + 1], c, -((r & 2 ? lj.w : lj.y) * kLog2e)));
+    if constexpr (part == 2) {
+      x[1][r] = x[0][r] * (x[1][r] - (r & 2 ? dj.z : dj.x));
+      x[1][r + 1] = x[0][r + 1] * (x[1][r + 1] - (r & 2 ? dj.w : dj.y));
+    }
+    if constexpr (part == 3) {
+      set_pair(pb[r >> 3], (r & 7) >> 1, cvt2h(x[0][r], x[0][r + 1]));
+      set_pair(sb[r >> 3], (r & 7) >> 1, cvt2h(x[1][r], x[1][r + 1]));
+    }
+  };
+  // keys past the query (in blocks up to the wavefront's own): P = dS = 0
+  auto mask = [&](int b, f32x16 (&x)[2]) {
+    const int d = kTok * (b - wave) - (lane & 31) + 4 * (lane >> 5);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) x[0][r] = acc_row(r, 0) + d < 0 ? -__builtin_inff() : x[0][r];
+  };
+  constexpr int NS = 2 * KC, NV = 4 * DT, half = NV / 2;  // MFMAs of S and dP, of dV and dK
+  constexpr int kPer = 32 / (NS + NV);                    // parts of P and dS per MFMA
+  constexpr int kHead = half * kPer;  // parts done in the block before (the last in this one's end)
+  constexpr int kAhead = 3;           // fragment reads issued ahead of their MFMAs
 
-  for (int q0 = kw0; q0 < L; q0 += kTok) {
-    __syncthreads();
-    sq.store(qsm, tid);
-    sd.store(dsm, tid);
-    if (tid < 2 * kTok) (tid < kTok ? lse_s : dl_s)[tid & (kTok - 1)] = lv;
-    __syncthreads();
-    load(q0 + kTok);  // the next block (past the sequence: zeros, not used)
-    if (q0 + kTok <= k0 || k0 >= L) continue;  // every query of the block precedes these keys
-    f32x16 s = f32x16{}, dp = f32x16{};
-#pragma unroll
-    for (int kk = 0; kk < KC; ++kk) {
-      const int row = lane & 31, ch = 2 * kk + (lane >> 5);
-      const half8_t qop = ld_tt<D>(qsm, row, ch), dop = ld_tt<D>(dsm, row, ch);
-      s = mfma(qop, kr[kk], s);
-      dp = mfma(dop, vr[kk], dp);
+  // Block b, its S and dP in x and the first kHead parts of its P and dS done: the next block's S
+  // and dP go to xn. last: there is none; masked: it may reach the diagonal.
+  auto block = [&](auto last, auto masked, int b, f32x16 (&x)[2], f32x16 (&xn)[2]) {
+    constexpr bool kLast = last.value;
+    sync_tile<NL>();  // block b + 1 landed, every wavefront is done with b - 1
+    if (!kLast) move_rows(b + 1);
+    tat.move(stage_at(b) - t_at);
+    t_at = stage_at(b);
+    const uint32_t at = row_at(b), atn = row_at(b + 1);
+    static_for<3>([&](auto j) { read_rows(std::integral_constant<int, j.value + 1>{}, at); });
+    if constexpr (!kLast) {
+      static_for<kAhead>([&](auto i) { read_r(i); });
+      __builtin_amdgcn_sched_barrier(0);
+      static_for<NS>([&](auto qc) {
+        constexpr int q = qc.value;
+        s_mfma(qc, xn);
+        if constexpr (q + kAhead < NS) read_r(std::integral_constant<int, q + kAhead>{});
+        else read_t(std::integral_constant<int, q + kAhead - NS>{});
+        static_for<kPer>([&](auto i) {
+          p_sub(std::integral_constant<int, kHead + q * kPer + i.value>{}, x);
+        });
+        if constexpr (q % 3 == 1 && q / 3 < NL) load(std::integral_constant<int, q / 3>{}, b + 3);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    } else {
+      static_for<kAhead>([&](auto i) { read_t(i); });
+      static_for<NS * kPer>([&](auto i) { p_sub(std::integral_constant<int, kHead + i.value>{}, x); });
+      __builtin_amdgcn_sched_barrier(0);
     }
-    // masks only where the block reaches the diagonal or the end of the sequence (uniform)
-    const bool edge = q0 < k0 + kTok || q0 + kTok > L;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int qr0 = 8 * j + 4 * (lane >> 5);
-      const float4 l4 = *reinterpret_cast<const float4*>(lse_s + qr0);
-      const float4 d4 = *reinterpret_cast<const float4*>(dl_s + qr0);
-      const float lq[4] = {l4.x, l4.y, l4.z, l4.w}, dq4[4] = {d4.x, d4.y, d4.z, d4.w};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = 4 * j + i;
-        s[r] = ex2(fmaf(s[r], c, -lq[i]));
-        if (edge) {
-          const int qq = q0 + qr0 + i;
-          s[r] = (qq < L && kj <= qq) ? s[r] : 0.f;
+    static_for<NV>([&](auto qc) {
+      constexpr int q = qc.value;
+      g_mfma(qc);
+      if constexpr (q + kAhead < NV) read_t(std::integral_constant<int, q + kAhead>{});
+      if constexpr (q < half) {
+        static_for<kPer>([&](auto i) {
+          p_sub(std::integral_constant<int, kHead + NS * kPer + q * kPer + i.value>{}, x);
+        });
+        if constexpr (!kLast && q == half - 1) {
+          read_rows(std::integral_constant<int, 0>{}, atn);
+          if constexpr (masked.value) mask(b + 1, xn);
         }
-        dp[r] = s[r] * (dp[r] - dq4[i]);
+      } else if constexpr (!kLast) {
+        static_for<kPer>([&](auto i) {
+          p_sub(std::integral_constant<int, (q - half) * kPer + i.value>{}, xn);
+        });
       }
-    }
-    half8_t pb[2], sb[2];
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      pb[kk] = to_b(s, kk);
-      sb[kk] = to_b(dp, kk);
-    }
-#pragma unroll
-    for (int u = 0; u < DT; ++u) {
-      const half8_t d0 = tr_operand<D>(dsm, 0, 32 * u, lane);
-      const half8_t d1 = tr_operand<D>(dsm, 16, 32 * u, lane);
-      const half8_t q0op = tr_operand<D>(qsm, 0, 32 * u, lane);
-      const half8_t q1op = tr_operand<D>(qsm, 16, 32 * u, lane);
-      dv[u] = mfma(d0, pb[0], dv[u]);
-      dk[u] = mfma(q0op, sb[0], dk[u]);
-      dv[u] = mfma(d1, pb[1], dv[u]);
-      dk[u] = mfma(q1op, sb[1], dk[u]);
-    }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  static_assert(3 * (NL - 1) + 1 < NS, "a block's loads are issued behind S and dP");
+  static_assert(kHead <= 16, "the parts done ahead need the first four queries' lse only");
+
+  sync_tile<2 * NL>();  // block 0 landed
+  move_rows(0);
+  static_for<NS>([&](auto i) { read_r(i); });
+  static_for<NS>([&](auto q) { s_mfma(q, s); });
+  read_rows(std::integral_constant<int, 0>{}, row_at(0));
+  mask(0, s);
+  static_for<kHead>([&](auto i) { p_sub(i, s); });
+  const std::false_type no;
+  const std::true_type yes;
+  int b = 0;
+  // the blocks of the diagonal, then the others, in pairs (no product changes its registers); a
+  // block that is left over
+  for (; b + 1 < min(kKeyWaves, nb - 1); b += 2) {
+    block(no, yes, b, s, sn);
+    block(no, yes, b + 1, sn, s);
   }
+  for (; b + 2 < nb; b += 2) {
+    block(no, no, b, s, sn);
+    block(no, no, b + 1, sn, s);
+  }
+  if (b + 1 < nb) {
+    block(no, yes, b, s, sn);
+    s[0] = sn[0];
+    s[1] = sn[1];
+    ++b;
+  }
+  block(yes, no, b, s, sn);
+  __builtin_amdgcn_s_waitcnt(0);  // loads past the sequence: none in flight when the wavefront ends
   if (kj < L) {
     const int64_t off = (int64_t)(start + kj) * qs + h * D;
     store_token_row<D>(a.dk + off, dk, a.scale, lane);
@@ -940,35 +1104,6 @@ int check_common(int32_t nseq, int32_t max_len, int64_t n, int32_t HQ, int32_t K
   // buffer offsets within one sequence's rows (plus the prefetch past its end) fit 32 bits
   QLORA_CHECK_ARG(((int64_t)max_len + 4 * kKB) * HQ * D * 2 < (1ll << 31));
   return 0;
-}
-
-// MODE: 1 dQ reading delta, 2 dQ forming delta
-template <int D, int G, int MODE>
-void launch_q(const Args& a, dim3 grid, hipStream_t s) {
-  if constexpr (MODE == 1)
-    hipLaunchKernelGGL((attn_dq_kernel<D, G, false>), grid, dim3(64 * G), 0, s, a);
-  else
-    hipLaunchKernelGGL((attn_dq_kernel<D, G, true>), grid, dim3(64 * G), 0, s, a);
-}
-
-template <int MODE, int D>
-void launch_q_g(const Args& a, int G, dim3 grid, hipStream_t s) {
-  switch (G) {
-    case 1: launch_q<D, 1, MODE>(a, grid, s); break;
-    case 2: launch_q<D, 2, MODE>(a, grid, s); break;
-    case 3: launch_q<D, 3, MODE>(a, grid, s); break;
-    case 4: launch_q<D, 4, MODE>(a, grid, s); break;
-    case 5: launch_q<D, 5, MODE>(a, grid, s); break;
-    case 6: launch_q<D, 6, MODE>(a, grid, s); break;
-    case 7: launch_q<D, 7, MODE>(a, grid, s); break;
-    default: launch_q<D, 8, MODE>(a, grid, s); break;
-  }
-}
-
-template <int MODE>
-void launch_q_any(const Args& a, int D, int G, dim3 grid, hipStream_t s) {
-  if (D == 128) launch_q_g<MODE, 128>(a, G, grid, s);
-  else launch_q_g<MODE, 64>(a, G, grid, s);
 }
 
 // Chunks of the split forms: chunk_keys a positive multiple of 64, at most kMaxChunks chunks.
@@ -1068,6 +1203,19 @@ bool bwd_concurrent(int32_t max_len, unsigned dq_groups) {
   return max_len >= 512 && dq_groups <= 320;
 }
 
+// The dQ kernel, OWN: forming delta itself.
+template <bool OWN>
+int launch_dq(Args a, int D, int32_t nseq, int64_t tiles, int64_t nch, hipStream_t s) {
+  constexpr int NW = 4;
+  a.ntiles = (int)qlora_cdiv(tiles * (a.HQ / a.KH), NW);
+  unsigned gx;
+  if (int rc = grid_of(a.ntiles, (int64_t)nseq * a.KH, &gx)) return rc;
+  const dim3 grid(gx, 1, (unsigned)nch), block(64 * NW);
+  if (D == 128) hipLaunchKernelGGL((attn_dq_kernel<128, NW, OWN>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((attn_dq_kernel<64, NW, OWN>), grid, block, 0, s, a);
+  return qlora_launch_status();
+}
+
 void launch_dkdv(const Args& b, int D, unsigned gkv, hipStream_t s) {
   if (D == 128)
     hipLaunchKernelGGL(attn_dkdv_kernel<128>, dim3(gkv), dim3(64 * kKeyWaves), 0, s, b);
@@ -1081,12 +1229,10 @@ int run_bwd(Args a, int32_t nseq, int32_t max_len, int D, int64_t nch, hipStream
   unsigned gkv;
   if (int rc = grid_of(b.ntiles, (int64_t)nseq * a.HQ, &gkv)) return rc;
   a.ntiles = (int)qlora_cdiv(max_len, kTok);
-  const int W = a.HQ / a.KH;
   unsigned gx;
   if (int rc = grid_of(a.ntiles, (int64_t)nseq * a.KH, &gx)) return rc;
   if (!bwd_concurrent(max_len, gx * (unsigned)nch)) {  // dQ (writing delta), then dK/dV
-    launch_q_any<2>(a, D, W, dim3(gx, 1, (unsigned)nch), s);
-    if (int rc = qlora_launch_status()) return rc;
+    if (int rc = launch_dq<true>(a, D, nseq, a.ntiles, nch, s)) return rc;
     if (nch > 1) {
       if (int rc = launch_merge<false>(a, D, nseq, nch, s)) return rc;
     }
@@ -1111,10 +1257,7 @@ int run_bwd(Args a, int32_t nseq, int32_t max_len, int D, int64_t nch, hipStream
   if (hipError_t e = hipStreamWaitEvent(ss->stream, ss->fork, 0)) return (int)e;
   launch_dkdv(b, D, gkv, ss->stream);
   int rc = qlora_launch_status();
-  if (rc == 0) {
-    launch_q_any<1>(a, D, W, dim3(gx, 1, (unsigned)nch), s);
-    rc = qlora_launch_status();
-  }
+  if (rc == 0) rc = launch_dq<false>(a, D, nseq, a.ntiles, nch, s);
   if (rc == 0 && nch > 1) rc = launch_merge<false>(a, D, nseq, nch, s);
   // join whatever was launched, also after an error
   if (hipError_t e = hipEventRecord(ss->join, ss->stream)) return rc ? rc : (int)e;

@@ -97,6 +97,13 @@ __device__ __forceinline__ void dma16(rsrc_t r, uint32_t voff, uint32_t lds) {
                : "scc");
 }
 
+// One DMA instruction of 4 bytes a lane to LDS byte lds (wave-uniform) + 4 lane.
+__device__ __forceinline__ void dma4(rsrc_t r, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+               :
+               : "s"(lds), "v"(voff), "s"(r));
+}
+
 // s_waitcnt with vmcnt(VM) and lgkmcnt(0), then s_barrier: this thread's LDS stores and all
 // but its VM most recent vector-memory loads are done, and so are every other thread's.
 template <int VM>

@@ -199,3 +199,13 @@ def test_forward_rescales_as_scores_grow(pkg, HQ, KH, D, lengths):
         assert (out[sl].float() - ref).abs().amax() < 2 * 2 ** -11
         torch.testing.assert_close(lse[:, sl], torch.logsumexp(s, -1), rtol=1e-5, atol=1e-4)
         start += x
+
+
+@pytest.mark.parametrize("HQ,KH,D", [(12, 2, 128), (14, 2, 64), (3, 3, 128)])
+@pytest.mark.parametrize("chunk", [0, 64])
+def test_backward_pipeline_block_counts(pkg, HQ, KH, D, chunk):
+    """One to eight 32-token blocks, whole and ragged: the backward kernels' first block, pairs,
+    left-over and last block, on and past the diagonal of a 128-key workgroup, and workgroups
+    whose last (query tile, q head) pairs lie past the sequence; key ranges whole and cut."""
+    _run(pkg, [32, 64, 95, 96, 97, 128, 129, 160, 161, 192, 224, 255, 256], HQ, KH, D, seed=chunk,
+         chunk=chunk)
