@@ -130,3 +130,33 @@ def test_ce_grad_equals_whole_row_kernel(pkg):
         g = logits[:, v0:v0 + 4096].clone()
         pkg.ops._ce_grad(g, targets, state, v0, n_sup)
         assert torch.equal(g[:n_sup].view(torch.int16), whole[:n_sup, v0:v0 + 4096].view(torch.int16))
+
+
+@pytest.mark.parametrize("rows,V", [(600, 4104), (1027, 16384), (300, 40960), (257, 90008),
+                                    (255, 131072), (515, 151936), (256, 172048)])
+def test_rows_in_registers_match_rows_read_twice(pkg, rows, V):
+    """Rows held in registers (every register block count) against the kernel that reads a row
+    twice, which takes rows that are not 16-byte aligned: equal bit for bit, masked columns
+    (-inf), ties and targets in the first and the last column among them."""
+    torch.manual_seed(V)
+    x = torch.randn(rows, V, device=DEV, dtype=torch.float16) * 3
+    targets = torch.randint(0, V, (rows,), device=DEV)
+    targets[::7] = -100
+    targets[1], targets[-1] = 0, V - 1
+    x[2, 5] = x[2, V - 9] = 60000.0  # a tie: the first column is the best
+    targets[2] = 5
+    x[3] = float("-inf")
+    x[3, V // 2] = 1.0
+    for zero in (True, False):
+        out = []
+        for pad in (0, 1):
+            buf = torch.zeros(rows, V + pad, device=DEV, dtype=torch.float16)
+            buf[:, :V] = x
+            view = buf[:, :V]
+            stats = [torch.empty(rows, device=DEV) for _ in range(2)]
+            stats.append(torch.empty(rows, device=DEV, dtype=torch.int32))
+            pkg.ops._ce(view, targets, *stats, zero_unsupervised=zero)
+            out.append([view, *stats])
+        for a, b in zip(*out):
+            assert torch.equal(a, b)
+        assert int(out[0][3][2]) == 1
