@@ -166,19 +166,19 @@ __device__ __forceinline__ void store_token_row_f32(float* row, const f32x16 (&a
 // cycles of the matrix core, beside 130 VALU instructions, 32 of them exponentials), so a block's
 // softmax is formed two values at a time behind the MFMAs of the next block's S and of P V (every
 // instruction pinned behind an MFMA by sched_barrier), no address is formed per fragment
-// (RowFrags, TrFrags), masks are applied from the diagonal on only, and the running maximum is
-// only a reference: it moves (and O is rescaled) when a score exceeds it by more than 2^8, so p <=
-// 2^8 and most blocks never rescale. K and V arrive by LDS DMA, two stages each, one barrier a
-// block. MI355X, 12/2 heads of 128, against one q head group per workgroup with the blocks staged
-// through registers and two barriers a block: four sequences of 283-997 tokens 36 -> 24 us, two of
-// 4,096 and 3,001 165 -> 100.
+// (RowFrags, TrFrags), and masks are applied from the diagonal on only. The maximum is the running
+// one of all scores so far, so a query's largest probability is 1, which fp16 holds exactly: with a
+// maximum that may lag (O rescaled only once a score exceeds it by 2^8) the forward is 3-5 % faster,
+// but every probability is rounded and the output's error against 64 bits 2-3 % larger. K and V
+// arrive by LDS DMA, two stages each, one barrier a block. MI355X, 12/2 heads of 128, against one q
+// head group per workgroup with the blocks staged through registers and two barriers a block (calls
+// in a stream of calls): four sequences of 283-997 tokens 36.5 -> 24.3 us, two of 4,096 and 3,001
+// 149 -> 107.
 // NW 4 or 8: four wavefronts spread a small batch over the CUs (24 us against 31 for those four
 // sequences); once 2,048 tiles fill all of them eight read K and V half as often (4,096 + 3,001,
 // forward and backward: 574 -> 560 us).
 // grid (ceil(ceil(max_len / 32) G / NW) nseq KH, 1, chunks), block 64 NW.
 // ------------------------------------------------------------------------------------------------
-constexpr float kRescale = 8.f;  // log2 units
-
 // max(a, b, c) without the quieting of signalling NaNs that fmaxf adds per operand.
 __device__ __forceinline__ float max3(float a, float b, float c) {
   float r;
@@ -358,7 +358,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_fwd_kernel(Args a) {
                 qr);
   f32x16 o[DT], s[2], sn[2];
   half8_t pb[4];
-  float m, mx, lsum = 0.f;
+  float m, mx, alpha = 1.f, lsum = 0.f, ps = 0.f;
   const float c = a.scale * kLog2e;
 #pragma unroll
   for (int u = 0; u < DT; ++u) o[u] = f32x16{};
@@ -396,7 +396,8 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_fwd_kernel(Args a) {
     constexpr int kk = ic.value >> 2, e = 2 * (ic.value & 3);
     const float p0 = ex2(fmaf(x[kk >> 1][8 * (kk & 1) + e], c, -m));
     const float p1 = ex2(fmaf(x[kk >> 1][8 * (kk & 1) + e + 1], c, -m));
-    lsum += p0 + p1;
+    ps += p0;
+    ps += p1;
     uint4 w = __builtin_bit_cast(uint4, pb[kk]);
     (e == 0 ? w.x : e == 2 ? w.y : e == 4 ? w.z : w.w) = cvt2h(p0, p1);
     pb[kk] = __builtin_bit_cast(half8_t, w);
@@ -417,12 +418,10 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_fwd_kernel(Args a) {
     v_at = v_lds(cur);
     if (!kLast) static_for<kAhead>([&](auto i) { read_k(i); });
     else static_for<kAhead>([&](auto i) { read_v(i); });
-    const bool grow = mx * c > m + kRescale;
-    if (__any(grow)) {
-      const float mn = grow ? mx * c : m;
-      const float alpha = grow ? ex2(m - mn) : 1.0f;
-      m = mn;
-      lsum *= alpha;
+    const float mn = fmaxf(m, mx * c);
+    alpha = ex2(m - mn);
+    m = mn;
+    if (__any(alpha != 1.f)) {  // once the running maxima settle, many blocks skip this
 #pragma unroll
       for (int u = 0; u < DT; ++u)
 #pragma unroll
@@ -476,6 +475,8 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_fwd_kernel(Args a) {
       }
       __builtin_amdgcn_sched_barrier(0);
     });
+    lsum = lsum * alpha + ps;
+    ps = 0.f;
     if constexpr (!kLast) {
       mx = pair_max(mx);
       cur = next;

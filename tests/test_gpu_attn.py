@@ -209,3 +209,31 @@ def test_backward_pipeline_block_counts(pkg, HQ, KH, D, chunk):
     whose last (query tile, q head) pairs lie past the sequence; key ranges whole and cut."""
     _run(pkg, [32, 64, 95, 96, 97, 128, 129, 160, 161, 192, 224, 255, 256], HQ, KH, D, seed=chunk,
          chunk=chunk)
+
+
+@pytest.mark.parametrize("HQ,KH,D", [(12, 2, 128), (14, 2, 64)])
+@pytest.mark.parametrize("chunk", [0, 128])
+def test_largest_probability_is_exact(pkg, HQ, KH, D, chunk):
+    """A query's largest probability is 1 whichever block of keys holds it. Key 64 (the second
+    block's first) is the maximum of every later query by 0.4 to 8 log2 units and alone has a
+    non-zero v, so O = v / l is rounded by the fp16 store only: half an ulp, and 2^-18 of it for
+    fp32's sums and reciprocal. A maximum that lags behind key 64 would round that probability to
+    fp16 too."""
+    n, top = 320, 64
+    scale = D ** -0.5
+    q, k, v = (torch.zeros(n, h, D, device=DEV, dtype=torch.float16) for h in (HQ, KH, KH))
+    lead = torch.linspace(0.4, 8.0, HQ, device=DEV)  # log2 units by which key 64 leads, per head
+    q[:, :, 0] = lead.half()
+    k[top, :, 0] = 1.0 / (scale * 1.4426950408889634)
+    g = torch.Generator(device=DEV).manual_seed(9)
+    v[top] = (1 + torch.rand(KH, D, device=DEV, generator=g)).half()
+    packed = _Packed([n])
+    packed._attn_plans = {("fwd", HQ, KH): chunk}
+    print(f"attn largest probability HQ={HQ} D={D} chunk={chunk}", flush=True)
+    out, _, _, _ = pkg.ops._attn_fwd(q, k, v, packed, scale)
+    s = q[0, :, 0].double() * k[top, 0, 0].double() * scale  # [HQ]: key 64's score; the others 0
+    rows = torch.arange(top, n, device=DEV, dtype=torch.float64)
+    weight = 1 / (1 + rows[:, None] * torch.exp(-s))  # [rows, HQ]; `rows` keys of score 0
+    exact = weight[:, :, None] * _expand(v[top:top + 1], HQ // KH).double()
+    ulp = torch.exp2(torch.floor(torch.log2(exact)) - 10)
+    assert ((out[top:].double() - exact).abs() <= ulp / 2 + exact * 2 ** -18).all()
