@@ -353,12 +353,14 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_fwd_kernel(Args a) {
   const int qi = q0 + (lane & 31), lim = min(qi, L - 1);
   const int nch = num_chunks(blocks_of(fc), a.chunk);
   const bool live = f < total && ch < nch;
+  // the wavefront's blocks end here
+  const int kbw = __builtin_amdgcn_readfirstlane(live ? min(blocks_of(fc), kb1) : kb0);
   half8_t qr[KC];  // queries past the sequence read zeros (their rows are not stored)
   load_token<D>(rows_rsrc(a.q + (int64_t)start * qs + h * D, L, qs, D), qi, (int)(qs * 2), lane,
                 qr);
   f32x16 o[DT], s[2], sn[2];
   half8_t pb[4];
-  float m, mx, alpha = 1.f, lsum = 0.f, ps = 0.f;
+  float m = 0.f, mx = 0.f, alpha = 1.f, lsum = 0.f, ps = 0.f;
   const float c = a.scale * kLog2e;
 #pragma unroll
   for (int u = 0; u < DT; ++u) o[u] = f32x16{};
@@ -405,8 +407,17 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_fwd_kernel(Args a) {
 
   int cur = 0;                                // the stage of K(b) and V(b); b + 1's is the other
   uint32_t k_at = k_lds(0), v_at = v_lds(0);  // the stages kat and vat address
+  // The loads of K(b + 2) and V(b + 1), when every wavefront is done with b - 1.
+  auto load = [&]() {
+    static_for<NI>([&](auto j) {
+      kd.template issue<j.value>(ksrc, k_lds(cur), wave);
+      vd.template issue<j.value>(vsrc, v_lds(cur ^ 1), wave);
+    });
+    kd.step(blk_b);
+    vd.step(blk_b);
+  };
   // Block b: its scores (masked) in x and their maximum in mx; the next block's go to xn and mx.
-  // last: there is none; masked: the next block reaches past the first query.
+  // last: there is none for this wavefront; masked: the next block reaches past the first query.
   auto block = [&](auto last, auto masked, int b, f32x16 (&x)[2], f32x16 (&xn)[2]) {
     constexpr bool kLast = last.value;
     const int next = cur ^ 1;
@@ -449,6 +460,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_fwd_kernel(Args a) {
       kd.step(blk_b);
       vd.step(blk_b);
     } else {
+      if (b + 1 < kb1) load();
       static_for<12>([&](auto i) { p_step(i, x); });
     }
     // P V: behind the first half of its products the rest of the probabilities, behind the second
@@ -477,37 +489,45 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_fwd_kernel(Args a) {
     });
     lsum = lsum * alpha + ps;
     ps = 0.f;
-    if constexpr (!kLast) {
-      mx = pair_max(mx);
-      cur = next;
-    }
+    if constexpr (!kLast) mx = pair_max(mx);
+    cur = next;
   };
 
-  // the first block's scores and maximum
   sync_tile<2 * NI>();  // K(kb0) landed
-  static_for<2 * KC>([&](auto i) { read_k(i); });
-  static_for<2 * KC>([&](auto q) { s_mfma(q, s); });
-  // max3 is assembly: the products' latency is waited for here
-  asm volatile("s_nop 15\n\ts_nop 15" : "+v"(s[0]), "+v"(s[1]));
-  mask(s, kb0 * kKB);
-  static_for<16>([&](auto i) { max_step(i, s); });
-  mx = pair_max(mx);
-  m = mx * c;
-  // masked from the first block that reaches past the first query on
   int b = kb0;
-  const int edge = min(q0 / kKB, kb1 - 1);
-  const std::false_type no;
-  const std::true_type yes;
-  for (; b + 2 < edge; b += 2) {  // in pairs: no score changes its registers
-    block(no, no, b, s, sn);
-    block(no, no, b + 1, sn, s);
+  if (b < kbw) {
+    // the first block's scores and maximum
+    static_for<2 * KC>([&](auto i) { read_k(i); });
+    static_for<2 * KC>([&](auto q) { s_mfma(q, s); });
+    // max3 is assembly: the products' latency is waited for here
+    asm volatile("s_nop 15\n\ts_nop 15" : "+v"(s[0]), "+v"(s[1]));
+    mask(s, kb0 * kKB);
+    static_for<16>([&](auto i) { max_step(i, s); });
+    mx = pair_max(mx);
+    m = mx * c;
+    // masked from the first block that reaches past the first query on
+    const int edge = min(q0 / kKB, kbw - 1);
+    const std::false_type no;
+    const std::true_type yes;
+    for (; b + 2 < edge; b += 2) {  // in pairs: no score changes its registers
+      block(no, no, b, s, sn);
+      block(no, no, b + 1, sn, s);
+    }
+    for (; b + 1 < kbw; ++b) {
+      block(no, yes, b, s, sn);
+      s[0] = sn[0];
+      s[1] = sn[1];
+    }
+    block(yes, no, b, s, sn);
+    ++b;
   }
-  for (; b + 1 < kb1; ++b) {
-    block(no, yes, b, s, sn);
-    s[0] = sn[0];
-    s[1] = sn[1];
+  // Blocks past the wavefront's own: loaded for the others. (Their P would be 0, but 0 times a
+  // value that is not finite is NaN: it may not reach queries before its key's block.)
+  for (; b < kb1; ++b) {
+    sync_tile<0>();
+    if (b + 1 < kb1) load();
+    cur ^= 1;
   }
-  block(yes, no, b, s, sn);
   __builtin_amdgcn_s_waitcnt(0);  // loads past the range: none in flight when the wavefront ends
   const float ltot = lsum + __shfl_xor(lsum, 32, 64);
   if (!live || qi >= L) return;
@@ -652,6 +672,8 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dq_kernel(Args a) {
   const int qi = q0 + (lane & 31), lim = min(qi, L - 1);
   const int nch = num_chunks(blocks_of(fc), a.chunk);
   const bool live = f < total && ch < nch;
+  // the wavefront's blocks end here
+  const int kbw = __builtin_amdgcn_readfirstlane(live ? min(blocks_of(fc), kb1) : kb0);
 
   // this query's q and dO (queries past the sequence read zeros; their dq is not stored), its
   // log-sum-exp and delta (attn_delta_kernel)
@@ -712,7 +734,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dq_kernel(Args a) {
   constexpr int kAhead = 3;  // fragment reads issued ahead of their MFMAs
 
   // Block b, its S and dP in x and the first steps of its dS done: the next block's go to xn.
-  // last: there is none; masked: it reaches past the first query.
+  // last: there is none for this wavefront; masked: it reaches past the first query.
   auto block = [&](auto last, auto masked, int b, f32x16 (&x)[2], f32x16 (&xn)[2]) {
     constexpr bool kLast = last.value;
     sync_tile<NL>();  // block b + 1 landed, every wavefront is done with b - 1
@@ -737,6 +759,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dq_kernel(Args a) {
         __builtin_amdgcn_sched_barrier(0);
       });
     } else {
+      if (b + 1 < kb1) static_for<NL>([&](auto j) { load(j, b + 3); });
       static_for<kAhead>([&](auto i) { read_t(i); });
       static_for<ds_before<D>(half + NS) - ds_before<D>(half)>([&](auto i) {
         ds_step(std::integral_constant<int, ds_before<D>(half) + i.value>{}, x);
@@ -766,24 +789,32 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dq_kernel(Args a) {
   static_assert(ds_before<D>(half + NS) >= 4, "the first 16 keys' dS is whole before dQ");
 
   sync_tile<2 * NL>();  // the first block landed
-  static_for<NS>([&](auto i) { read_r(i); });
-  static_for<NS>([&](auto q) { s_mfma(q, s); });
-  mask(kb0, s);
-  static_for<ds_before<D>(half)>([&](auto i) { ds_step(i, s); });
-  const std::false_type no;
-  const std::true_type yes;
   int b = kb0;
-  const int edge = min(q0 / kTok, kb1 - 1);
-  for (; b + 2 < edge; b += 2) {  // in pairs: no product changes its registers
-    block(no, no, b, s, sn);
-    block(no, no, b + 1, sn, s);
+  if (b < kbw) {
+    static_for<NS>([&](auto i) { read_r(i); });
+    static_for<NS>([&](auto q) { s_mfma(q, s); });
+    mask(kb0, s);
+    static_for<ds_before<D>(half)>([&](auto i) { ds_step(i, s); });
+    const std::false_type no;
+    const std::true_type yes;
+    const int edge = min(q0 / kTok, kbw - 1);
+    for (; b + 2 < edge; b += 2) {  // in pairs: no product changes its registers
+      block(no, no, b, s, sn);
+      block(no, no, b + 1, sn, s);
+    }
+    for (; b + 1 < kbw; ++b) {
+      block(no, yes, b, s, sn);
+      s[0] = sn[0];
+      s[1] = sn[1];
+    }
+    block(yes, no, b, s, sn);
+    ++b;
   }
-  for (; b + 1 < kb1; ++b) {
-    block(no, yes, b, s, sn);
-    s[0] = sn[0];
-    s[1] = sn[1];
+  // blocks past the wavefront's own: loaded for the others (as the forward)
+  for (; b < kb1; ++b) {
+    sync_tile<NL>();
+    static_for<NL>([&](auto j) { load(j, b + 3); });
   }
-  block(yes, no, b, s, sn);
   __builtin_amdgcn_s_waitcnt(0);  // loads past the range: none in flight when the wavefront ends
   if (!live || qi >= L) return;
   if (nch == 1) {
@@ -866,8 +897,9 @@ __global__ __launch_bounds__(32 * D / 4) void attn_merge_kernel(Args a) {
 // time (p_sub) behind the MFMAs of block b + 1's S and dP and of block b's dV and dK, every
 // instruction pinned behind an MFMA by sched_barrier. Per block and wavefront 32 MFMAs (D = 128;
 // 1,024 cycles of the matrix core) stand beside about 150 VALU instructions. Q and dO arrive by LDS
-// DMA, four stages (two blocks' time to land), one barrier a block; rows past the sequence read
-// zeros, which add nothing, so only the first four blocks (the diagonal) are masked.
+// DMA, four stages (two blocks' time to land), one barrier a block. A wavefront skips the query
+// blocks before its keys; its first block (the diagonal) and its last (rows past the sequence, which
+// read zeros) are masked, the others run without.
 // MI355X, 12/2 heads of 128, against two barriers a block, staging through registers and a block's
 // products, exponentials and products one after the other: two sequences of 4,096 and 3,001 tokens
 // 290 -> 216 us, four of 283-997 58 -> 43.
@@ -972,13 +1004,20 @@ __global__ __launch_bounds__(64 * kKeyWaves, 1) void attn_dkdv_kernel(Args a) {
     l4[j.value] = __builtin_bit_cast(float4, *(lds_f4_t*)(uintptr_t)(at + 32 * j.value));
     d4[j.value] = __builtin_bit_cast(float4, *(lds_f4_t*)(uintptr_t)(at + 256 + 32 * j.value));
   };
-  // Part k % 4 of the P and dS of queries acc_row(2 (k / 4)) and the next (k = 0 .. 31)
-  auto p_sub = [&](auto kc, f32x16 (&x)[2]) {
+  // Part k % 4 of the P and dS of queries acc_row(2 (k / 4)) and the next (k = 0 .. 31) of block b.
+  // masked: P = 0 where the query precedes the key or lies past the sequence, also where its score or
+  // log-sum-exp is not finite.
+  auto p_sub = [&](auto masked, auto kc, int b, f32x16 (&x)[2]) {
     constexpr int r = 2 * (kc.value >> 2), part = kc.value & 3;
     const float4 lj = l4[r >> 2], dj = d4[r >> 2];
-    if constexpr (part == 0) x[0][r] = ex2(fmaf(x[0][r], c, -((r & 2 ? lj.z : lj.x) * kLog2e)));
-    if constexpr (part == 1)
-      x[0][r + 1] = ex2(fmaf(x[0][r + 1], c, -((r & 2 ? lj.w : lj.y) * kLog2e)));
+    auto p_of = [&](int i, float lse) {
+      const float p = ex2(fmaf(x[0][i], c, -(lse * kLog2e)));
+      if constexpr (!masked.value) return p;
+      const int first = kj - kw0 - kTok * b - 4 * (lane >> 5);  // the key's own query
+      return acc_row(i, 0) >= first && acc_row(i, 0) - first < L - kj ? p : 0.f;
+    };
+    if constexpr (part == 0) x[0][r] = p_of(r, r & 2 ? lj.z : lj.x);
+    if constexpr (part == 1) x[0][r + 1] = p_of(r + 1, r & 2 ? lj.w : lj.y);
     if constexpr (part == 2) {
       x[1][r] = x[0][r] * (x[1][r] - (r & 2 ? dj.z : dj.x));
       x[1][r + 1] = x[0][r + 1] * (x[1][r + 1] - (r & 2 ? dj.w : dj.y));
@@ -988,19 +1027,13 @@ __global__ __launch_bounds__(64 * kKeyWaves, 1) void attn_dkdv_kernel(Args a) {
       set_pair(sb[r >> 3], (r & 7) >> 1, cvt2h(x[1][r], x[1][r + 1]));
     }
   };
-  // keys past the query (in blocks up to the wavefront's own): P = dS = 0
-  auto mask = [&](int b, f32x16 (&x)[2]) {
-    const int d = kTok * (b - wave) - (lane & 31) + 4 * (lane >> 5);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) x[0][r] = acc_row(r, 0) + d < 0 ? -__builtin_inff() : x[0][r];
-  };
   constexpr int NS = 2 * KC, NV = 4 * DT, half = NV / 2;  // MFMAs of S and dP, of dV and dK
   constexpr int kPer = 32 / (NS + NV);                    // parts of P and dS per MFMA
   constexpr int kHead = half * kPer;  // parts done in the block before (the last in this one's end)
   constexpr int kAhead = 3;           // fragment reads issued ahead of their MFMAs
 
   // Block b, its S and dP in x and the first kHead parts of its P and dS done: the next block's S
-  // and dP go to xn. last: there is none; masked: it may reach the diagonal.
+  // and dP go to xn. last: there is none; masked: one of the two may need masks.
   auto block = [&](auto last, auto masked, int b, f32x16 (&x)[2], f32x16 (&xn)[2]) {
     constexpr bool kLast = last.value;
     sync_tile<NL>();  // block b + 1 landed, every wavefront is done with b - 1
@@ -1018,14 +1051,16 @@ __global__ __launch_bounds__(64 * kKeyWaves, 1) void attn_dkdv_kernel(Args a) {
         if constexpr (q + kAhead < NS) read_r(std::integral_constant<int, q + kAhead>{});
         else read_t(std::integral_constant<int, q + kAhead - NS>{});
         static_for<kPer>([&](auto i) {
-          p_sub(std::integral_constant<int, kHead + q * kPer + i.value>{}, x);
+          p_sub(masked, std::integral_constant<int, kHead + q * kPer + i.value>{}, b, x);
         });
         if constexpr (q % 3 == 1 && q / 3 < NL) load(std::integral_constant<int, q / 3>{}, b + 3);
         __builtin_amdgcn_sched_barrier(0);
       });
     } else {
       static_for<kAhead>([&](auto i) { read_t(i); });
-      static_for<NS * kPer>([&](auto i) { p_sub(std::integral_constant<int, kHead + i.value>{}, x); });
+      static_for<NS * kPer>([&](auto i) {
+        p_sub(masked, std::integral_constant<int, kHead + i.value>{}, b, x);
+      });
       __builtin_amdgcn_sched_barrier(0);
     }
     static_for<NV>([&](auto qc) {
@@ -1034,15 +1069,12 @@ __global__ __launch_bounds__(64 * kKeyWaves, 1) void attn_dkdv_kernel(Args a) {
       if constexpr (q + kAhead < NV) read_t(std::integral_constant<int, q + kAhead>{});
       if constexpr (q < half) {
         static_for<kPer>([&](auto i) {
-          p_sub(std::integral_constant<int, kHead + NS * kPer + q * kPer + i.value>{}, x);
+          p_sub(masked, std::integral_constant<int, kHead + NS * kPer + q * kPer + i.value>{}, b, x);
         });
-        if constexpr (!kLast && q == half - 1) {
-          read_rows(std::integral_constant<int, 0>{}, atn);
-          if constexpr (masked.value) mask(b + 1, xn);
-        }
+        if constexpr (!kLast && q == half - 1) read_rows(std::integral_constant<int, 0>{}, atn);
       } else if constexpr (!kLast) {
         static_for<kPer>([&](auto i) {
-          p_sub(std::integral_constant<int, (q - half) * kPer + i.value>{}, xn);
+          p_sub(masked, std::integral_constant<int, (q - half) * kPer + i.value>{}, b + 1, xn);
         });
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -1052,32 +1084,40 @@ __global__ __launch_bounds__(64 * kKeyWaves, 1) void attn_dkdv_kernel(Args a) {
   static_assert(kHead <= 16, "the parts done ahead need the first four queries' lse only");
 
   sync_tile<2 * NL>();  // block 0 landed
-  move_rows(0);
-  static_for<NS>([&](auto i) { read_r(i); });
-  static_for<NS>([&](auto q) { s_mfma(q, s); });
-  read_rows(std::integral_constant<int, 0>{}, row_at(0));
-  mask(0, s);
-  static_for<kHead>([&](auto i) { p_sub(i, s); });
-  const std::false_type no;
-  const std::true_type yes;
+  // blocks wholly before the wavefront's keys: loaded for the others (their P would be 0, but 0
+  // times a value that is not finite is NaN: it may not reach later keys)
   int b = 0;
-  // the blocks of the diagonal, then the others, in pairs (no product changes its registers); a
-  // block that is left over
-  for (; b + 1 < min(kKeyWaves, nb - 1); b += 2) {
-    block(no, yes, b, s, sn);
-    block(no, yes, b + 1, sn, s);
+  for (; b < min(wave, nb); ++b) {
+    sync_tile<NL>();
+    static_for<NL>([&](auto j) { load(j, b + 3); });
   }
-  for (; b + 2 < nb; b += 2) {
-    block(no, no, b, s, sn);
-    block(no, no, b + 1, sn, s);
+  if (b < nb) {
+    const std::false_type no;
+    const std::true_type yes;
+    move_rows(b);
+    static_for<NS>([&](auto i) { read_r(i); });
+    static_for<NS>([&](auto q) { s_mfma(q, s); });
+    read_rows(std::integral_constant<int, 0>{}, row_at(b));
+    static_for<kHead>([&](auto i) { p_sub(yes, i, b, s); });
+    // the diagonal's block, the blocks without masks in pairs (no product changes its registers),
+    // those that are left over and the last
+    if (b + 1 < nb) {
+      block(no, yes, b, s, sn);
+      s[0] = sn[0];
+      s[1] = sn[1];
+      ++b;
+    }
+    for (; b + 3 < nb; b += 2) {
+      block(no, no, b, s, sn);
+      block(no, no, b + 1, sn, s);
+    }
+    for (; b + 1 < nb; ++b) {
+      block(no, yes, b, s, sn);
+      s[0] = sn[0];
+      s[1] = sn[1];
+    }
+    block(yes, yes, b, s, sn);
   }
-  if (b + 1 < nb) {
-    block(no, yes, b, s, sn);
-    s[0] = sn[0];
-    s[1] = sn[1];
-    ++b;
-  }
-  block(yes, no, b, s, sn);
   __builtin_amdgcn_s_waitcnt(0);  // loads past the sequence: none in flight when the wavefront ends
   if (kj < L) {
     const int64_t off = (int64_t)(start + kj) * qs + h * D;

@@ -237,3 +237,58 @@ def test_largest_probability_is_exact(pkg, HQ, KH, D, chunk):
     exact = weight[:, :, None] * _expand(v[top:top + 1], HQ // KH).double()
     ulp = torch.exp2(torch.floor(torch.log2(exact)) - 10)
     assert ((out[top:].double() - exact).abs() <= ulp / 2 + exact * 2 ** -18).all()
+
+
+@pytest.mark.parametrize("HQ,KH,D,lengths,chunk",
+                         [(1, 1, 128, [700], 0), (14, 2, 64, [500, 333], 0),
+                          (12, 2, 128, [700, 300], 128), (8, 8, 64, [601], 64),
+                          (8, 8, 64, [4096, 3000, 2000], 0), (8, 8, 128, [4096, 3000, 2000], 256)])
+def test_values_that_are_not_finite_stay_causal(pkg, HQ, KH, D, lengths, chunk):
+    """A token's infinities and NaNs reach other tokens' rows only where the sums over its own block
+    multiply them by a probability of 0: queries before its key block (64 keys forward, 32 dQ) and
+    keys after its query block (32) keep their bits, whatever else their workgroup holds (four and
+    eight wavefronts, 1 to 7 q heads a kv head, whole and cut key ranges). A score of -inf masks its
+    key: that key's dK and dV are 0, also in a ragged last block."""
+    g = torch.Generator(device=DEV).manual_seed(3)
+    n, last = sum(lengths), lengths[0] - 1
+    q = torch.rand(n, HQ, D, device=DEV, generator=g).half()
+    k, v = (torch.randn(n, KH, D, device=DEV, generator=g).half() for _ in range(2))
+    dout = torch.randn(n, HQ, D, device=DEV, generator=g).half()
+
+    def run(**changed):
+        t = dict(dict(q=q, k=k, v=v, dout=dout), **changed)
+        packed = _Packed(lengths)
+        packed._attn_plans = {("fwd", HQ, KH): chunk, ("dq", HQ, KH): chunk}
+        out, lse, _, _ = pkg.ops._attn_fwd(t["q"], t["k"], t["v"], packed, D ** -0.5)
+        dq, dk, dv = pkg.ops._attn_bwd(t["dout"], t["q"], t["k"], t["v"], out, lse, None, None,
+                                       packed, D ** -0.5)
+        torch.cuda.synchronize()
+        return out, lse, dq, dk, dv
+
+    def with_(x, at, value):
+        y = x.clone()
+        y[at, :, 3] = value
+        return y
+
+    inf, nan = float("inf"), float("nan")
+    out, lse, dq, dk, dv = run()
+    for at in (130, 160, 255, last):
+        print(f"attn not finite HQ={HQ} KH={KH} D={D} lengths={lengths} chunk={chunk} at={at}",
+              flush=True)
+        before64, before32 = at // 64 * 64, at // 32 * 32
+        for value in (inf, nan):
+            o, l, q_, _, _ = run(v=with_(v, at, value))
+            assert torch.equal(o[:before64], out[:before64]), ("V", value)
+            assert torch.equal(l, lse)
+            assert torch.equal(q_[:before64], dq[:before64])  # delta is formed from out
+            _, _, _, k_, v_ = run(dout=with_(dout, at, value))
+            assert torch.equal(k_[at // 32 * 32 + 32:], dk[at // 32 * 32 + 32:]), ("dO", value)
+            assert torch.equal(v_[at // 32 * 32 + 32:], dv[at // 32 * 32 + 32:]), ("dO", value)
+            _, _, _, k_, v_ = run(q=with_(q, at, value))
+            assert torch.equal(k_[at // 32 * 32 + 32:], dk[at // 32 * 32 + 32:]), ("Q", value)
+            assert torch.equal(v_[at + 1:], dv[at + 1:]), ("Q", value)
+        o, _, q_, k_, v_ = run(k=with_(k, at, -inf))  # q > 0: the key's scores are -inf
+        assert torch.isfinite(o).all() and torch.equal(o[:at], out[:at])
+        assert torch.equal(q_[:before32], dq[:before32])
+        assert not k_[at].any() and not v_[at].any()
+        assert torch.isfinite(k_).all() and torch.isfinite(v_).all()
