@@ -341,7 +341,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_fwd_kernel(Args a) {
     kd.step(blk_b);
   };
   dma_k(0);
-  dma_k(1);
+  if (kb0 + 1 < kb1) dma_k(1);
   static_for<NI>([&](auto j) { vd.template issue<j.value>(vsrc, v_lds(0), wave); });
   vd.step(blk_b);
 
@@ -356,8 +356,9 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_fwd_kernel(Args a) {
   // the wavefront's blocks end here
   const int kbw = __builtin_amdgcn_readfirstlane(live ? min(blocks_of(fc), kb1) : kb0);
   half8_t qr[KC];  // queries past the sequence read zeros (their rows are not stored)
-  load_token<D>(rows_rsrc(a.q + (int64_t)start * qs + h * D, L, qs, D), qi, (int)(qs * 2), lane,
-                qr);
+  if (live)
+    load_token<D>(rows_rsrc(a.q + (int64_t)start * qs + h * D, L, qs, D), qi, (int)(qs * 2), lane,
+                  qr);
   f32x16 o[DT], s[2], sn[2];
   half8_t pb[4];
   float m = 0.f, mx = 0.f, alpha = 1.f, lsum = 0.f, ps = 0.f;
@@ -493,7 +494,8 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_fwd_kernel(Args a) {
     cur = next;
   };
 
-  sync_tile<2 * NI>();  // K(kb0) landed
+  if (kb0 + 1 < kb1) sync_tile<2 * NI>();  // K(kb0) landed
+  else sync_tile<NI>();
   int b = kb0;
   if (b < kbw) {
     // the first block's scores and maximum
@@ -603,6 +605,14 @@ struct PairDma {
   }
 };
 
+// The wait for the first of `blocks` blocks, up to three of them in flight (NL loads each): a block
+// that is not there is not loaded, and its loads do not count.
+template <int NL>
+__device__ __forceinline__ void first_block(int blocks) {
+  if (blocks >= 3) sync_tile<2 * NL>();
+  else sync_tile<0>();
+}
+
 // Halves 2 i and 2 i + 1 of a fragment.
 __device__ __forceinline__ void set_pair(half8_t& f, int i, uint32_t pair) {
   uint4 w = __builtin_bit_cast(uint4, f);
@@ -663,7 +673,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dq_kernel(Args a) {
     dma.template issue<j.value>(ksrc, vsrc, stage_at(b), wave);
     if constexpr (j.value == NL - 1) dma.d.step((uint32_t)(kTok * kvs_b));
   };
-  for (int b = kb0; b < kb0 + 3; ++b) static_for<NL>([&](auto j) { load(j, b); });
+  for (int b = kb0; b < min(kb0 + 3, kb1); ++b) static_for<NL>([&](auto j) { load(j, b); });
 
   // the wavefront's tile, as the forward: past the last tile the last one again, not stored
   const int f = grp * NW + wave, fc = min(f, total - 1);
@@ -679,24 +689,25 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dq_kernel(Args a) {
   // log-sum-exp and delta (attn_delta_kernel)
   const int64_t hoff = (int64_t)start * qs + h * D;
   half8_t qr[KC], dr[KC];
-  load_token<D>(rows_rsrc(a.q + hoff, L, qs, D), qi, qs_b, lane, qr);
-  load_token<D>(rows_rsrc(a.dout + hoff, L, qs, D), qi, qs_b, lane, dr);
-  const float lse2 =
-      buf_load_f32(make_rsrc(a.lse + (int64_t)h * a.n + start, (uint32_t)L * 4), qi * 4) *
-      kLog2e;
-  float delta;
-  if constexpr (OWN_DELTA) {
-    half8_t orow[KC];
-    load_token<D>(rows_rsrc(a.o + hoff, L, qs, D), qi, qs_b, lane, orow);
-    float dpart = 0.f;
+  float lse2 = 0.f, delta = 0.f;
+  if (live) {
+    load_token<D>(rows_rsrc(a.q + hoff, L, qs, D), qi, qs_b, lane, qr);
+    load_token<D>(rows_rsrc(a.dout + hoff, L, qs, D), qi, qs_b, lane, dr);
+    lse2 = buf_load_f32(make_rsrc(a.lse + (int64_t)h * a.n + start, (uint32_t)L * 4), qi * 4) *
+           kLog2e;
+    if constexpr (OWN_DELTA) {
+      half8_t orow[KC];
+      load_token<D>(rows_rsrc(a.o + hoff, L, qs, D), qi, qs_b, lane, orow);
+      float dpart = 0.f;
 #pragma unroll
-    for (int kk = 0; kk < KC; ++kk)
+      for (int kk = 0; kk < KC; ++kk)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) dpart += (float)dr[kk][i] * (float)orow[kk][i];
-    delta = dpart + __shfl_xor(dpart, 32, 64);
-    if (live && ch == 0 && qi < L && lane < 32) a.delta[(int64_t)h * a.n + start + qi] = delta;
-  } else {
-    delta = buf_load_f32(make_rsrc(a.delta + (int64_t)h * a.n + start, (uint32_t)L * 4), qi * 4);
+        for (int i = 0; i < 8; ++i) dpart += (float)dr[kk][i] * (float)orow[kk][i];
+      delta = dpart + __shfl_xor(dpart, 32, 64);
+      if (ch == 0 && qi < L && lane < 32) a.delta[(int64_t)h * a.n + start + qi] = delta;
+    } else {
+      delta = buf_load_f32(make_rsrc(a.delta + (int64_t)h * a.n + start, (uint32_t)L * 4), qi * 4);
+    }
   }
 
   f32x16 dq[DT], s[2], sn[2];  // s: S and dP
@@ -788,7 +799,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dq_kernel(Args a) {
   static_assert(3 * (NL - 1) + 1 < NS, "a block's loads are issued behind S and dP");
   static_assert(ds_before<D>(half + NS) >= 4, "the first 16 keys' dS is whole before dQ");
 
-  sync_tile<2 * NL>();  // the first block landed
+  first_block<NL>(kb1 - kb0);
   int b = kb0;
   if (b < kbw) {
     static_for<NS>([&](auto i) { read_r(i); });
@@ -952,10 +963,11 @@ __global__ __launch_bounds__(64 * kKeyWaves, 1) void attn_dkdv_kernel(Args a) {
       row_off += kTok * 4;
     }
   };
-  for (int b = 0; b < 3; ++b) static_for<NL>([&](auto j) { load(j, b); });
+  // with fewer than three blocks only those there are (first_block)
+  for (int b = 0; b < min(3, nb); ++b) static_for<NL>([&](auto j) { load(j, b); });
 
   half8_t kr[KC], vr[KC];  // keys past the sequence read zeros (their rows are not stored)
-  {
+  if (wave < nb) {         // (a wavefront of such keys only multiplies nothing)
     const int64_t koff = (int64_t)start * kvs + kvh * D;
     load_token<D>(rows_rsrc(a.k + koff, L, kvs, D), kj, kvs_b, lane, kr);
     load_token<D>(rows_rsrc(a.v + koff, L, kvs, D), kj, kvs_b, lane, vr);
@@ -1083,7 +1095,7 @@ __global__ __launch_bounds__(64 * kKeyWaves, 1) void attn_dkdv_kernel(Args a) {
   static_assert(3 * (NL - 1) + 1 < NS, "a block's loads are issued behind S and dP");
   static_assert(kHead <= 16, "the parts done ahead need the first four queries' lse only");
 
-  sync_tile<2 * NL>();  // block 0 landed
+  first_block<NL>(nb);
   // blocks wholly before the wavefront's keys: loaded for the others (their P would be 0, but 0
   // times a value that is not finite is NaN: it may not reach later keys)
   int b = 0;
