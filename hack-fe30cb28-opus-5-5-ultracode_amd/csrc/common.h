@@ -94,14 +94,15 @@ __device__ __forceinline__ void dma16(rsrc_t r, uint32_t voff, uint32_t lds) {
   asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds"
                :
                : "s"(lds), "n"(1024 * J), "v"(voff), "s"(r)
-               : "scc");
+               : "scc", "m0", "memory");
 }
 
 // One DMA instruction of 4 bytes a lane to LDS byte lds (wave-uniform) + 4 lane.
 __device__ __forceinline__ void dma4(rsrc_t r, uint32_t voff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
                :
-               : "s"(lds), "v"(voff), "s"(r));
+               : "s"(lds), "v"(voff), "s"(r)
+               : "m0", "memory");
 }
 
 // s_waitcnt with vmcnt(VM) and lgkmcnt(0), then s_barrier: this thread's LDS stores and all
@@ -109,8 +110,10 @@ __device__ __forceinline__ void dma4(rsrc_t r, uint32_t voff, uint32_t lds) {
 template <int VM>
 __device__ __forceinline__ void sync_tile() {
   static_assert(VM >= 0 && VM < 64, "vmcnt is 6 bits");
+  asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | (7 << 4));
   __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
 }
 
 // f(0), f(1), .. f(N - 1), each index a compile-time constant.
