@@ -174,9 +174,8 @@ __device__ __forceinline__ void store_token_row_f32(float* row, const f32x16 (&a
 // head group per workgroup with the blocks staged through registers and two barriers a block (calls
 // in a stream of calls): four sequences of 283-997 tokens 36.5 -> 24.3 us, two of 4,096 and 3,001
 // 149 -> 107.
-// NW 4 or 8: four wavefronts spread a small batch over the CUs (24 us against 31 for those four
-// sequences); once 2,048 tiles fill all of them eight read K and V half as often (4,096 + 3,001,
-// forward and backward: 574 -> 560 us).
+// NW 4 or 8 (wide_groups): four wavefronts spread a small batch over the CUs, eight read K and V half
+// as often.
 // grid (ceil(ceil(max_len / 32) G / NW) nseq KH, 1, chunks), block 64 NW.
 // ------------------------------------------------------------------------------------------------
 // max(a, b, c) without the quieting of signalling NaNs that fmaxf adds per operand.
@@ -1093,7 +1092,8 @@ __global__ __launch_bounds__(64 * kKeyWaves, 1) void attn_dkdv_kernel(Args a) {
     });
   };
   static_assert(3 * (NL - 1) + 1 < NS, "a block's loads are issued behind S and dP");
-  static_assert(kHead <= 16, "the parts done ahead need the first four queries' lse only");
+  static_assert(kHead <= 8, "the parts done ahead need the first four queries' lse only");
+  static_assert(kPer * (NS + NV) == 32, "every part of P and dS has its place");
 
   first_block<NL>(nb);
   // blocks wholly before the wavefront's keys: loaded for the others (their P would be 0, but 0
@@ -1206,18 +1206,28 @@ int launch_fwd(Args a, int32_t nseq, int64_t tiles, int64_t nch, hipStream_t s) 
   return qlora_launch_status();
 }
 
-// Whether the (query or key tile, head) pairs fill the GPU with workgroups of eight wavefronts.
-bool wide_groups(const Args& a) { return qlora_cdiv(a.n, kTok) * a.HQ >= 2048; }
+// Whether the forward takes workgroups of eight wavefronts: from 3,072 (query tile, head) pairs on,
+// 1.5 of such workgroups a CU. Four against eight, MI355X, head counts 8/8 to 64/8, us: below, four
+// are faster by 0-20 % (12/2 heads of 128, six sequences of 1,024, 2,304 pairs: 32 against 35; 8/8,
+// 8,192 tokens, 2,048: 166 against 194); above, within 5 % either way for most (12/2, two of 4,096:
+// 121.5 against 122.7; 14/2 heads of 64, 4,096 + 3,001, 3,108: 76 against 70; 32/32, 4,096, 4,096:
+// 163 against 148; 64/8 heads of 64, 4,096, 8,192: 171 against 176). Also where four would need more
+// workgroups than a grid holds.
+bool wide_groups(const Args& a, int32_t nseq, int64_t tiles) {
+  return qlora_cdiv(a.n, kTok) * a.HQ >= 3072 ||
+         qlora_cdiv(tiles * (a.HQ / a.KH), 4) * nseq * a.KH >= (1ll << 31);
+}
 
 int run_fwd(Args a, int32_t nseq, int32_t max_len, int D, int64_t nch, hipStream_t s) {
   const int64_t tiles = qlora_cdiv(max_len, kTok);
+  const bool wide = wide_groups(a, nseq, tiles);
   int rc;
   if (D == 128)
-    rc = wide_groups(a) ? launch_fwd<128, 8>(a, nseq, tiles, nch, s)
-                        : launch_fwd<128, 4>(a, nseq, tiles, nch, s);
+    rc = wide ? launch_fwd<128, 8>(a, nseq, tiles, nch, s)
+              : launch_fwd<128, 4>(a, nseq, tiles, nch, s);
   else
-    rc = wide_groups(a) ? launch_fwd<64, 8>(a, nseq, tiles, nch, s)
-                        : launch_fwd<64, 4>(a, nseq, tiles, nch, s);
+    rc = wide ? launch_fwd<64, 8>(a, nseq, tiles, nch, s)
+              : launch_fwd<64, 4>(a, nseq, tiles, nch, s);
   a.ntiles = (int)tiles;
   if (rc == 0 && nch > 1) rc = launch_merge<true>(a, D, nseq, nch, s);
   return rc;

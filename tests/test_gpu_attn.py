@@ -171,10 +171,10 @@ def test_concurrent_backward_other_shapes(pkg, HQ, KH, D):
 
 
 @pytest.mark.parametrize("HQ,KH,D,lengths", [(12, 2, 128, [700, 33]), (14, 2, 64, [700, 33]),
-                                             (12, 2, 128, [1500, 1200, 1100, 1000, 900])])
+                                             (12, 2, 128, [2500, 1700, 1600, 1500, 1000])])
 def test_forward_rescales_as_scores_grow(pkg, HQ, KH, D, lengths):
     """Scores that grow along the keys by far more than 2^8 move the forward's reference maximum
-    (and rescale O) in block after block; four and eight wavefronts a workgroup (2,048 tiles and
+    (and rescale O) in block after block; four and eight wavefronts a workgroup (3,072 tiles and
     more). Against fp32 SDPA on the GPU; out is a convex combination of v (|v| <= 1 here), p and
     out are rounded to fp16 once each: 2 x 2^-11 of it."""
     g = torch.Generator(device=DEV).manual_seed(5)
@@ -242,7 +242,7 @@ def test_largest_probability_is_exact(pkg, HQ, KH, D, chunk):
 @pytest.mark.parametrize("HQ,KH,D,lengths,chunk",
                          [(1, 1, 128, [700], 0), (14, 2, 64, [500, 333], 0),
                           (12, 2, 128, [700, 300], 128), (8, 8, 64, [601], 64),
-                          (8, 8, 64, [4096, 3000, 2000], 0), (8, 8, 128, [4096, 3000, 2000], 256)])
+                          (8, 8, 64, [4096, 4000, 4300], 0), (8, 8, 128, [4096, 4000, 4300], 320)])
 def test_values_that_are_not_finite_stay_causal(pkg, HQ, KH, D, lengths, chunk):
     """A token's infinities and NaNs reach other tokens' rows only where the sums over its own block
     multiply them by a probability of 0: queries before its key block (64 keys forward, 32 dQ) and
@@ -292,3 +292,40 @@ def test_values_that_are_not_finite_stay_causal(pkg, HQ, KH, D, lengths, chunk):
         assert torch.equal(q_[:before32], dq[:before32])
         assert not k_[at].any() and not v_[at].any()
         assert torch.isfinite(k_).all() and torch.isfinite(v_).all()
+
+
+@pytest.mark.parametrize("HQ,KH,D,lengths", [(14, 2, 64, [2600, 1, 33, 2100, 65, 2400, 7]),
+                                             (8, 8, 128, [3300, 64, 1, 5000, 31, 4000, 130]),
+                                             (28, 4, 128, [1900, 1, 65, 1600, 33, 97])])
+def test_eight_wavefronts_match_four(pkg, HQ, KH, D, lengths):
+    """3,072 (query tile, head) pairs and more take workgroups of eight wavefronts; each sequence on
+    its own takes four, with the same bits: long sequences beside very short and ragged ones, so that
+    workgroups end in wavefronts without a tile and hold tiles of different lengths. The longest
+    sequence against fp32 SDPA."""
+    assert -(-sum(lengths) // 32) * HQ >= 3072 > -(-max(lengths) // 32) * HQ
+    g = torch.Generator(device=DEV).manual_seed(HQ)
+    n = sum(lengths)
+    q = torch.randn(n, HQ, D, device=DEV, generator=g).half()
+    k, v = (torch.randn(n, KH, D, device=DEV, generator=g).half() for _ in range(2))
+
+    def run(lengths, sl):
+        packed = _Packed(lengths)
+        packed._attn_plans = {("fwd", HQ, KH): 0}
+        return pkg.ops._attn_fwd(q[sl], k[sl], v[sl], packed, D ** -0.5)[:2]
+
+    print(f"attn eight wavefronts HQ={HQ} KH={KH} D={D} lengths={lengths}", flush=True)
+    out, lse = run(lengths, slice(0, n))
+    start = 0
+    for x in lengths:
+        sl = slice(start, start + x)
+        o, l = run([x], sl)
+        assert torch.equal(out[sl], o) and torch.equal(lse[:, sl], l), x
+        if x == max(lengths):
+            qf, kf, vf = (t[sl].float().transpose(0, 1) for t in (q, _expand(k, HQ // KH),
+                                                                  _expand(v, HQ // KH)))
+            s = torch.bmm(qf, kf.transpose(1, 2).contiguous()) * D ** -0.5
+            s = s.masked_fill(torch.ones(x, x, device=DEV, dtype=torch.bool).triu(1),
+                              float("-inf"))
+            close(o, torch.bmm(torch.softmax(s, -1), vf).transpose(0, 1), 2e-3)
+            close(l, torch.logsumexp(s, -1), 1e-4)
+        start += x
