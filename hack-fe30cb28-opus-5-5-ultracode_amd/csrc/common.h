@@ -87,6 +87,10 @@ __device__ __forceinline__ void buf_store16(rsrc_t r, uint32_t off, uint4 v) {
 }
 
 // ---- LDS DMA ---------------------------------------------------------------------------------------
+// (the compiler warns that M0 is reserved: it is, and the clobber keeps it from reusing a value of its
+// own across the statement)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 // One DMA instruction (16 bytes a lane) to LDS byte lds (wave-uniform) + 1024 J + 16 lane. The
 // caller waits for it (sync_tile).
 template <int J>
@@ -104,6 +108,7 @@ __device__ __forceinline__ void dma4(rsrc_t r, uint32_t voff, uint32_t lds) {
                : "s"(lds), "v"(voff), "s"(r)
                : "m0", "memory");
 }
+#pragma clang diagnostic pop
 
 // s_waitcnt with vmcnt(VM) and lgkmcnt(0), then s_barrier: this thread's LDS stores and all
 // but its VM most recent vector-memory loads are done, and so are every other thread's.
