@@ -823,52 +823,42 @@ def _attn_shapes(q, k, v, packed):
     return q.shape[0], q.shape[1], k.shape[1], q.shape[2], cu, dev
 
 
-# Split of the attention's key ranges (qlora_attn_fwd_split / qlora_attn_bwd_split). Resident
-# workgroups of the forward and dQ kernels: one per CU (their registers), 256 on an MI355X. A
-# workgroup costs about two key blocks of fixed work (loads of its queries, the first block, the
-# stores) plus one per block it walks (5.2 us for one 64-key block, +1.75 us per block, with few
-# workgroups running). Measured on MI355X: with a sequence of 1024 (64 workgroups) chunks of 256
-# keys take the forward from 35.7 to 25.8 us and dQ + dK/dV from 115 to 92 us, with one of 2048
-# chunks of 512 keys 65.6 -> 53.3 and 212 -> 191 us; once the unsplit launch fills half the GPU
-# (four sequences of up to 1024 tokens: 166 workgroups) every split was slower (each workgroup's
-# key blocks take longer when more run at once, and the merge costs 8-12 us), so none is made.
-ATTN_SLOTS = 256
-ATTN_WG_BLOCKS = 2.0
+# Split of the attention's key ranges (qlora_attn_fwd_split / qlora_attn_bwd_split): a launch of
+# few workgroups is as long as its longest key range, so that is cut into chunks, which cost a merge
+# launch (3-6 us) and the partials' round trip. The forward's and dQ's workgroups are four (query
+# tile, q head) pairs of a kv head; two fit a CU, 512 the GPU. Measured on MI355X over head counts 1/1
+# to 28/4 and sequences of 512-8,192 tokens, us a call:
+#   forward, up to 128 workgroups and sequences of 1,536 and more: 2,048 tokens, 8/8 heads of 128 (128
+#   workgroups) 35.8 -> 29.3, 4/4 (64) 34.7 -> 22.8; 4,096, 2/2 heads of 64 (64) 46.6 -> 22.5. From
+#   1,024 with heads of 128 and up to 64 workgroups, 4/4 (32) 20.1 -> 17.6; with heads of 64, 2/2 (16),
+#   15.6 -> 17.9. Fuller launches were slower cut: 12/2 heads of 128, 1,024 tokens (96) 20.9 -> 22.8,
+#   2,048 (192) 35.8 -> 36.2 at best, 4,096 (384) 76.5 -> 85.
+#   backward, up to 64 workgroups and sequences of 1,024 and more: 2/2 heads of 64, 1,024 tokens (16
+#   workgroups) 43.1 -> 37.3, 4,096 (64) 132 -> 106; 14/2, 1,024 (112) 43.4 -> 44.2; 4/4 heads of 128,
+#   1,024 (32) 58.5 -> 52.6. From 1,536 with heads of 128 the dK/dV kernel, which is not cut, is the
+#   longer one, and running it beside dQ hides more (8/8, 3,072: 114; cut, beside 122-132, in turn 138).
 ATTN_MAX_CHUNKS = 16
-ATTN_MIN_CHUNK = 256
 
 
-def attn_chunk(lengths, heads, block):
-    """Keys per workgroup (a multiple of 64) for the split kernels, or 0 for no split: none when
-    the unsplit launch already has half as many workgroups as the GPU holds, else the chunk of
-    at least ATTN_MIN_CHUNK keys that minimises max(longest workgroup, total work / resident
-    workgroups), over a batch of sequence `lengths`, `heads` (sequence, head) workgroup rows per
-    tile, key blocks of `block` keys (64: forward, 32: dQ)."""
-    lengths = [int(x) for x in lengths if x > 0]
-    if not lengths:
+def attn_chunk(lengths, HQ, KH, D, kind):
+    """Keys per workgroup (a multiple of 64) for the split kernels over a batch of sequence
+    `lengths`, or 0 for no split; kind "fwd" or "dq"."""
+    max_len = max(lengths, default=0)
+    groups = KH * sum(-(-(-(-x // 32) * (HQ // KH)) // 4) for x in lengths if x > 0)
+    long = max_len >= 1536
+    if kind == "fwd" and long:
+        most, smallest, slots = 128, 512, 384
+    elif max_len >= 1024 and not (long if D == 128 else kind == "fwd"):
+        most, smallest, slots = 64, 256, 256
+    else:
         return 0
-    max_len = max(lengths)
-    nkb = []
-    for L in lengths:  # tile t of 32 queries walks ceil(min(32 (t + 1), L) / block) blocks
-        nkb += [-(-min(32 * (t + 1), L) // block) for t in range(-(-L // 32))]
-    if len(nkb) * heads > ATTN_SLOTS // 2:
+    if groups > most:
         return 0
-    nkb = torch.tensor(nkb, dtype=torch.float64)
-    best, best_cost = 0, None
-    cands = [0] + [c for c in (256, 384, 512, 768, 1024, 1536, 2048, 3072, 4096, 6144, 8192)
-                   if c >= ATTN_MIN_CHUNK and c < max_len and -(-max_len // c) <= ATTN_MAX_CHUNKS]
-    for c in cands:
-        per = c // block if c else int(nkb.max())
-        nch = torch.ceil(nkb / per)
-        total = float((nch * ATTN_WG_BLOCKS + nkb).sum()) * heads
-        longest = ATTN_WG_BLOCKS + min(per, float(nkb.max())) + (0.3 * float(nch.max()) if c else 0)
-        cost = max(longest, total / ATTN_SLOTS)
-        if best_cost is None or cost < best_cost * 0.97:  # prefer fewer chunks on a near tie
-            best, best_cost = c, cost
-    return best
+    chunks = min(slots // groups, -(-max_len // smallest), ATTN_MAX_CHUNKS)
+    return -(-max_len // (64 * chunks)) * 64
 
 
-def _attn_plan(packed, kind, HQ, KH):
+def _attn_plan(packed, kind, HQ, KH, D):
     """Chunk keys for `kind` ("fwd", "dq") of this batch, computed once per packed batch from the
     host-side lengths (0 when there are none)."""
     plans = getattr(packed, "_attn_plans", None)
@@ -884,8 +874,7 @@ def _attn_plan(packed, kind, HQ, KH):
         if cu is None:
             plans[key] = 0
         else:
-            lengths = [b - a for a, b in zip(cu[:-1], cu[1:])]
-            plans[key] = attn_chunk(lengths, KH, 64 if kind == "fwd" else 32)
+            plans[key] = attn_chunk([b - a for a, b in zip(cu[:-1], cu[1:])], HQ, KH, D, kind)
     return plans[key]
 
 
@@ -906,7 +895,7 @@ def _attn_fwd(q, k, v, packed, scale):
     lse = torch.empty((HQ, n), device=dev, dtype=torch.float32)
     if n:
         nseq, max_len = cu.numel() - 1, int(packed.max_len)
-        chunk = _attn_plan(packed, "fwd", HQ, KH)
+        chunk = _attn_plan(packed, "fwd", HQ, KH, D)
         work = _attn_work(n, max_len, HQ, D, chunk, dev) if chunk else None
         _lib.call("qlora_attn_fwd_split", _ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lse),
                   _ptr(cu), nseq, max_len, n, HQ, KH, D, float(scale), chunk, _ptr(work),
@@ -931,7 +920,7 @@ def _attn_bwd(dout, q, k, v, out, lse, seed, offset, packed, scale):
     if n:
         nseq, max_len = cu.numel() - 1, int(packed.max_len)
         delta = torch.empty((HQ, n), device=dev, dtype=torch.float32)
-        chunk = _attn_plan(packed, "dq", HQ, KH)
+        chunk = _attn_plan(packed, "dq", HQ, KH, D)
         work = _attn_work(n, max_len, HQ, D, chunk, dev) if chunk else None
         _lib.call("qlora_attn_bwd_split", _ptr(dout), _ptr(q), _ptr(k), _ptr(v), _ptr(out),
                   _ptr(lse), _ptr(delta), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(cu), nseq, max_len,

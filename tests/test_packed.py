@@ -155,3 +155,24 @@ def test_gemm_shape_check():
                dict(hidden_size=1500)):
         with pytest.raises(E.UnsupportedModel, match="multiples of 128"):
             E.check_gemm_shapes(E.Qwen2Config(**kw))
+
+
+def test_attention_split_counts_the_launched_workgroups():
+    """Key ranges are cut only where the forward's (dQ's) workgroups, four (query tile, q head) pairs
+    of a kv head each, are few and long: the q heads of a kv head count too. Chunks are whole blocks
+    of 64 keys, at most 16."""
+    chunk = pkg.ops.attn_chunk
+    assert chunk([], 12, 2, 128, "fwd") == 0 and chunk([0, 0], 2, 2, 64, "dq") == 0
+    # the same tiles and kv heads, 96 and 16 workgroups
+    assert chunk([2048], 2, 2, 128, "fwd") == 512 and chunk([2048], 12, 2, 128, "fwd") == 0
+    assert chunk([2048], 8, 8, 128, "fwd") == 704 and chunk([2080], 8, 8, 128, "fwd") == 0
+    assert chunk([1535], 1, 1, 64, "fwd") == 0 and chunk([1536], 1, 1, 64, "fwd") == 512
+    assert chunk([1023], 4, 4, 128, "fwd") == 0 and chunk([1024], 4, 4, 128, "fwd") == 256
+    assert chunk([1024], 12, 2, 128, "fwd") == 0 and chunk([611, 997, 283, 744], 12, 2, 128, "fwd") == 0
+    assert chunk([4096], 1, 1, 128, "dq") == 0  # long with heads of 128: dK/dV beside dQ instead
+    assert chunk([1024], 4, 4, 128, "dq") == 256
+    assert chunk([1024], 2, 2, 64, "dq") == 256 and chunk([1024], 14, 2, 64, "dq") == 0
+    for n in range(1, 20000, 317):
+        for kind in ("fwd", "dq"):
+            c = chunk([n, 5], 2, 1, 64 + n % 2 * 64, kind)
+            assert c % 64 == 0 and (c == 0 or 2 <= -(-n // c) <= 16)
