@@ -63,7 +63,8 @@ struct Args {
   int64_t n;
   int HQ, KH;
   int chunk;             // key blocks per workgroup (0: the whole range in one workgroup)
-  int ntiles;            // query (forward, dQ) or key (dK/dV) tiles per sequence and head
+  int ntiles;            // workgroups per sequence and kv head (forward, dQ), per sequence and q
+                         // head (dK/dV); query tiles per sequence (merge)
   float scale;
 };
 
@@ -1259,11 +1260,16 @@ int side_stream(SideStream** out) {
   return 0;
 }
 
-// Concurrent dQ and dK/dV pay when the dQ launch is long but leaves most of the GPU idle (few
-// long sequences: at most ~1.25 workgroups per CU of 256, key ranges of 512 and more); a full
-// launch gains nothing from the second stream and pays the delta kernel and the fork.
-bool bwd_concurrent(int32_t max_len, unsigned dq_groups) {
-  return max_len >= 512 && dq_groups <= 320;
+// dQ and dK/dV side by side pay when one of them leaves room for the other (at most 300 dK/dV
+// workgroups, one a CU at D = 128) and both are long enough for the delta kernel, the fork and the
+// join. Side by side against in turn on MI355X, us a call: 12/2 heads of 128, 1,024 tokens (96
+// workgroups) 59 against 61, 512 (48) 48 against 41, 2,048 (192) 87 against 106, 3,072 (288) 141
+// against 160, four of 283-997 (384) 70 against 66, two of 2,048 (384) 139 against 125, 28/4, 1,536
+// (336) 104 against 95; 8/8 heads of 64, 2,048 (128) 71 against 74, 3,072 (192) 94 against 104, 14/2,
+// 2,048 (224) 77 against 75, 1,024 (112) 52 against 43. A cut dQ (nch chunks) runs in turn: it fills
+// the GPU itself.
+bool bwd_concurrent(int32_t max_len, int D, int64_t nch, unsigned dkdv_groups) {
+  return nch == 1 && max_len >= (D == 128 ? 1024 : 2560) && dkdv_groups <= 300;
 }
 
 // The dQ kernel, OWN: forming delta itself.
@@ -1291,10 +1297,8 @@ int run_bwd(Args a, int32_t nseq, int32_t max_len, int D, int64_t nch, hipStream
   b.ntiles = (int)qlora_cdiv(max_len, kTok * kKeyWaves);
   unsigned gkv;
   if (int rc = grid_of(b.ntiles, (int64_t)nseq * a.HQ, &gkv)) return rc;
-  a.ntiles = (int)qlora_cdiv(max_len, kTok);
-  unsigned gx;
-  if (int rc = grid_of(a.ntiles, (int64_t)nseq * a.KH, &gx)) return rc;
-  if (!bwd_concurrent(max_len, gx * (unsigned)nch)) {  // dQ (writing delta), then dK/dV
+  a.ntiles = (int)qlora_cdiv(max_len, kTok);  // of dQ and the merge
+  if (!bwd_concurrent(max_len, D, nch, gkv)) {  // dQ (writing delta), then dK/dV
     if (int rc = launch_dq<true>(a, D, nseq, a.ntiles, nch, s)) return rc;
     if (nch > 1) {
       if (int rc = launch_merge<false>(a, D, nseq, nch, s)) return rc;

@@ -164,10 +164,24 @@ def test_concurrent_backward_matches_sequential(pkg):
 
 @pytest.mark.parametrize("HQ,KH,D", [(14, 2, 64), (16, 2, 128), (28, 4, 128), (8, 8, 64)])
 def test_concurrent_backward_other_shapes(pkg, HQ, KH, D):
-    """The concurrent backward (few sequences, max_len >= 512: dK/dV beside dQ, delta from its
-    own kernel) at other head sizes and group counts (Qwen2 0.5B 14/2 x 64, 3B 16/2, 7B 28/4,
-    and one q head per kv head) against fp32 SDPA, key ranges unsplit."""
+    """The backward of few sequences at other head sizes and group counts (Qwen2 0.5B 14/2 x 64, 3B
+    16/2, 7B 28/4, and one q head per kv head) against fp32 SDPA, key ranges unsplit. (dQ and dK/dV
+    in turn: test_backward_rules runs them side by side.)"""
     _run(pkg, [600, 300], HQ, KH, D, seed=HQ + D, chunk=0)
+
+
+@pytest.mark.parametrize("HQ,KH,D,lengths,split", [
+    (16, 2, 128, [1024, 70], False), (28, 4, 128, [1050], False), (8, 8, 128, [1100, 1, 333], False),
+    (5, 5, 64, [2600], False), (14, 2, 64, [2560], False),  # dQ beside dK/dV, delta from its own kernel
+    (2, 2, 64, [1024, 33], True), (1, 1, 64, [1500, 1100], True), (4, 2, 64, [1030], True),
+    (4, 4, 128, [1024, 9], True)])
+def test_backward_rules(pkg, HQ, KH, D, lengths, split):
+    """The package's own choices on either side of their lines: dQ beside dK/dV (long sequences, few
+    dK/dV workgroups), dQ's and the forward's key ranges cut (fewer still); against fp32 SDPA."""
+    assert (pkg.ops.attn_chunk(lengths, HQ, KH, D, "dq") > 0) == split
+    groups = -(-max(lengths) // 128) * len(lengths) * HQ
+    assert split or (groups <= 300 and max(lengths) >= (1024 if D == 128 else 2560))
+    _run(pkg, lengths, HQ, KH, D, seed=HQ + D)
 
 
 @pytest.mark.parametrize("HQ,KH,D,lengths", [(12, 2, 128, [700, 33]), (14, 2, 64, [700, 33]),
