@@ -16,7 +16,8 @@ Beside it, on the same JSON line:
                  in backward (nothing but the input kept)
   keep_all       the same step with every layer keeping its intermediates (no recompute)
   roofline       the step's largest hand-written kernel by time, the package's MFMA GEMM
-                 (hgemm_kernel: the gate|up forward with the SwiGLU epilogue), 2 M N K flops
+                 (hgemm256_kernel and hgemm_kernel: the gate|up forward with the SwiGLU
+                 epilogue), 2 M N K flops
                  over the dispatch-recorded duration, against the fp16 MFMA peak, over the
                  launches of four extra untimed steps (four batches' token counts)
   roofline_dequant  the step's NF4 dequant launches (the north star's dequant GB/s)
@@ -234,9 +235,9 @@ def measure_step_kernels(pkg, trainer, batches, cfg):
             out.append(dict(r, kernel=name, traffic=None))
     mine = own.summary(select=lambda a: a[13] in P.SWIGLU_EPIS)
     if mine is not None:
-        mine = dict(mine, kernel="hgemm_kernel (qlora_gemm16): the gate|up forward with the "
-                                 "SwiGLU epilogue (and the [g|u] product kept for the backward), "
-                                 "this package's MFMA GEMM")
+        mine = dict(mine, kernel="hgemm256_kernel and hgemm_kernel (qlora_gemm16): the gate|up "
+                                 "forward with the SwiGLU epilogue (and the [g|u] product kept "
+                                 "for the backward), this package's MFMA GEMM")
     return mine, dq.summary(), out
 
 

@@ -29,8 +29,8 @@
 // staged Q/dO. The next tiles arrive by LDS DMA during the current tile's MFMAs. dK/dV come out
 // per q head ([n, HQ, D]); the caller sums each group (the RoPE backward does, as the reference
 // sums the repeated kv heads). The log-sum-exp of the forward (natural log, fp32 [HQ, n]) and
-// delta = rowsum(dO * O) (fp32 [HQ, n], written by attn_delta_kernel) feed the dQ and the dK/dV
-// kernels, which run at the same time on two streams.
+// delta = rowsum(dO * O) (fp32 [HQ, n], written by attn_delta_kernel or the dQ kernel) feed the dQ
+// and the dK/dV kernels, which run in turn or side by side on two streams (bwd_concurrent).
 #include "common.h"
 
 #include <mutex>
@@ -171,10 +171,10 @@ __device__ __forceinline__ void store_token_row_f32(float* row, const f32x16 (&a
 // one of all scores so far, so a query's largest probability is 1, which fp16 holds exactly: with a
 // maximum that may lag (O rescaled only once a score exceeds it by 2^8) the forward is 3-5 % faster,
 // but every probability is rounded and the output's error against 64 bits 2-3 % larger. K and V
-// arrive by LDS DMA, two stages each, one barrier a block. MI355X, 12/2 heads of 128, against one q
-// head group per workgroup with the blocks staged through registers and two barriers a block (calls
-// in a stream of calls): four sequences of 283-997 tokens 36.5 -> 24.3 us, two of 4,096 and 3,001
-// 149 -> 107.
+// arrive by LDS DMA, two stages each, one barrier a block. MI355X, against one q head group per
+// workgroup with the blocks staged through registers and two barriers a block, kernel averages: four
+// sequences of 283-997 tokens, 12/2 heads of 128, 37.0 -> 25.5 us, 14/2 of 64 24.9 -> 17.0; two of
+// 4,096 and 3,001 151 -> 113 and 103 -> 80.
 // NW 4 or 8 (wide_groups): four wavefronts spread a small batch over the CUs, eight read K and V half
 // as often.
 // grid (ceil(ceil(max_len / 32) G / NW) nseq KH, 1, chunks), block 64 NW.
@@ -634,8 +634,9 @@ constexpr int ds_before(int q) {
 // and the chunks as the forward. Block b's dS is formed a few instructions at a time (ds_step)
 // behind the MFMAs of block b + 1's S and dP and of block b's dQ, as in attn_dkdv_kernel; K and V
 // arrive by LDS DMA, four stages, one barrier a block, and masks start at the diagonal.
-// MI355X, 12/2 heads of 128, against one q head group per workgroup, staging through registers and
-// two barriers a block: sequences of 4,096 and 3,001 tokens 200 -> 143 us, four of 283-997 44 -> 34.
+// MI355X, against one q head group per workgroup, staging through registers and two barriers a block,
+// kernel averages: sequences of 4,096 and 3,001 tokens, 12/2 heads of 128, 194 -> 140 us, 14/2 of 64
+// 126 -> 91; four of 283-997 (beside dK/dV before, in turn now) 44 -> 31 and 27 -> 19.
 // OWN_DELTA: the kernel forms delta itself (lanes l and l ^ 32 sum the chunks of
 // attn_delta_kernel's two threads, in its order) and the first chunk writes it for the dK/dV
 // kernel that follows; else it reads attn_delta_kernel's.
@@ -911,9 +912,10 @@ __global__ __launch_bounds__(32 * D / 4) void attn_merge_kernel(Args a) {
 // DMA, four stages (two blocks' time to land), one barrier a block. A wavefront skips the query
 // blocks before its keys; its first block (the diagonal) and its last (rows past the sequence, which
 // read zeros) are masked, the others run without.
-// MI355X, 12/2 heads of 128, against two barriers a block, staging through registers and a block's
-// products, exponentials and products one after the other: two sequences of 4,096 and 3,001 tokens
-// 290 -> 216 us, four of 283-997 58 -> 43.
+// MI355X, against two barriers a block, staging through registers and a block's products,
+// exponentials and products one after the other, kernel averages: two sequences of 4,096 and 3,001
+// tokens, 12/2 heads of 128, 279 -> 212 us, 14/2 of 64 166 -> 129; four of 283-997 (beside dQ before,
+// in turn now) 66 -> 41 and 50 -> 29.
 // grid (nseq * HQ * ceil(max_len / 128)), block 256.
 // ------------------------------------------------------------------------------------------------
 constexpr int kKeyWaves = 4;

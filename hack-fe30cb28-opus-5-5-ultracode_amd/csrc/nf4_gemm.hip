@@ -1625,7 +1625,7 @@ bool al(const void* p, uintptr_t a) { return ((uintptr_t)p & (a - 1)) == 0; }
 
 constexpr int kCUs = 256;  // compute units of an MI355X
 
-// Workgroups resident at once for a tile shape: 256 x 256 tiles take a CU each (128 KB of
+// Workgroups resident at once for a tile shape: 256 x 256 tiles take a CU each (all 160 KB of
 // LDS), 128 x 128 tiles two per CU with two stages (64 KB each), one with four (128 KB).
 int64_t slots_of(int tile, int stages) { return tile == 128 && stages == 2 ? 2 * kCUs : kCUs; }
 
@@ -1660,7 +1660,12 @@ int64_t n_tiles_of(int64_t N, int epi, int tile) {
 // once: 256 tiles of 256 x 256, 512 of 128 x 128 with two stages, 256 with four); its cost is
 //   a rounds + b (the k elements its rounds walk) + c (MB of fp32 partials) + d (a reduce),
 // the constants (us) least-squares fits of every variant over the step's nine products and the
-// lm_head's at 1,024 - 4,096 tokens on MI355X (HIP graphs, warm caches; median error 5-8 %).
+// lm_head's at 1,024 - 4,096 tokens on MI355X (HIP graphs, warm caches). The fit is older than
+// hgemm256_kernel, which is 10-18 % faster than what the 256 x 256 row priced, and knows no fewer
+// than 1,024 rows. A fit to the present kernels by the same single-product timings (1,750 of them, the
+// choice within 0.4 % of the fastest there) was slower where products follow one another, their
+// operands and partials cold: the MLP block at 2,048 tokens, 1,536 x 8,960, forward and backward,
+// 406 us with that fit, 388 with this one.
 // Candidates: 256 x 256 tiles in 1-8 K slices (7 or 8 fill the GPU when a long reduction has
 // 32-36 output tiles), 128 x 128 tiles in 1, 2 or 4 (up to K = 12,288: beyond that the
 // measurements favoured 256 x 256 tiles, whose loads per flop are half).

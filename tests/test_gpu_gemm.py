@@ -570,3 +570,34 @@ def test_gemm_f32_against_fp64(pkg, mode, M, K):
     auto = L.gemm_f32(a, b, mode, alpha=0.25, row_scale=rs, resid=resid)
     assert (auto.double() - want).abs().max().item() <= 1e-5 * want.abs().max().item() + 1e-6
     assert torch.equal(auto, L.gemm_f32(a, b, mode, alpha=0.25, row_scale=rs, resid=resid))
+
+
+@pytest.mark.parametrize("mode,M,K", [(1, 1, 128), (1, 301, 384), (2, 256, 256)])
+@pytest.mark.parametrize("tile,stages", [(256, 2), (128, 2)])
+@pytest.mark.parametrize("where", ["out ld", "out base", "resid ld", "resid base"])
+def test_gemm_f32_rows_without_16_byte_alignment(pkg, mode, M, K, tile, stages, where):
+    """Output or residual rows that do not start on 16 bytes (an odd leading dimension, a base of 4
+    bytes) are stored by element: the bits of the aligned call, nothing written beside the output."""
+    L = pkg.linear
+    N = 512
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    a = (torch.randn(*((M, K) if mode == 1 else (K, M)), generator=g, device=DEV) * 0.5).half()
+    b = (torch.randn(K, N, generator=g, device=DEV) * 0.02).half()
+    resid = torch.randn(M, N, generator=g, device=DEV)
+    rs = torch.rand(M, generator=g, device=DEV) + 0.5
+
+    def view(name):  # [M, N] within a buffer of 7.0
+        buf = torch.full((M * (N + 1) + 4,), 7.0, device=DEV)
+        ld = N + 1 if where == name + " ld" else N
+        off = 1 if where == name + " base" else 0
+        return buf, buf[off:off + M * ld].view(M, ld)[:, :N]
+
+    want = L.gemm_f32(a, b, mode, alpha=0.25, row_scale=rs, resid=resid, tile=tile, stages=stages)
+    buf, out = view("out")
+    _, res = view("resid")
+    res.copy_(resid)
+    L.gemm_f32(a, b, mode, alpha=0.25, row_scale=rs, resid=res, out=out, tile=tile, stages=stages)
+    assert torch.equal(out, want)
+    assert int((buf != 7.0).sum()) <= M * N
+    out.fill_(7.0)
+    assert (buf == 7.0).all()
