@@ -143,23 +143,27 @@ __device__ __forceinline__ int tile_order(int b, int total) {
   return b < full ? (b % 8) * (full / 8) + b / 8 : b;
 }
 
-// Tile t of one K slice -> (M tile, N tile): M tiles in groups of at most 12 (the groups as even
-// as they go), a group's M tiles fastest, then the N tiles. An XCD works on 32 consecutive tiles
-// at a time, and what its L2 must bring in per k-tile is their M tiles plus their N tiles: with
-// all 16 M tiles of 4,001 rows fastest it is 16 + 2 operand blocks of 32 KB, in two groups of 8
-// it is 8 + 4 (the [4001, 3584] x [37888, 3584] SwiGLU product 1,039 -> 1,011 us). Up to 12 M
-// tiles (3,072 rows) one group is as good and reads B once.
-__device__ __forceinline__ void tile_pos_lane(int t, int m_tiles, int n_tiles, int& tm, int& tn) {
-  const int groups = (m_tiles + 11) / 12, gm = (m_tiles + groups - 1) / groups;
-  const int grp = t / (gm * n_tiles);
-  t -= grp * gm * n_tiles;
-  const int w = min(gm, m_tiles - grp * gm);
-  tm = grp * gm + t % w;
-  tn = t / w;
-}
-// The same for a wave-uniform t, in scalar registers.
-__device__ __forceinline__ void tile_pos(int t, int m_tiles, int n_tiles, int& tm, int& tn) {
-  tile_pos_lane(t, m_tiles, n_tiles, tm, tn);
+// Tile t of one K slice -> (M tile, N tile). The first `cols` N tiles are taken with their M tiles
+// in groups of at most 12 (the groups as even as they go), a group's M tiles fastest, then the N
+// tiles; the tiles past those columns (of a launch whose last tiles run as K slices: the column that
+// is cut, and the slices' tiles) N tile by N tile, M fastest, so the sliced tiles are the last ones
+// column by column however the others are grouped. An XCD works on 32 consecutive tiles at a time,
+// and what its L2 must bring in per k-tile is their M tiles plus their N tiles: with all 16 M tiles
+// of 4,001 rows fastest it is 16 + 2 operand blocks of 32 KB, in two groups of 8 it is 8 + 4 (the
+// [4001, 3584] x [37888, 3584] SwiGLU product 1,039 -> 1,011 us). Up to 12 M tiles (3,072 rows) one
+// group is as good and reads B once. t is wave-uniform, the result in scalar registers.
+__device__ __forceinline__ void tile_pos(int t, int m_tiles, int cols, int& tm, int& tn) {
+  if (t < m_tiles * cols) {
+    const int groups = (m_tiles + 11) / 12, gm = (m_tiles + groups - 1) / groups;
+    const int grp = t / (gm * cols);
+    t -= grp * gm * cols;
+    const int w = min(gm, m_tiles - grp * gm);
+    tm = grp * gm + t % w;
+    tn = t / w;
+  } else {
+    tm = t % m_tiles;
+    tn = t / m_tiles;
+  }
   tm = __builtin_amdgcn_readfirstlane(tm);
   tn = __builtin_amdgcn_readfirstlane(tn);
 }
@@ -168,13 +172,14 @@ __device__ __forceinline__ void tile_pos(int t, int m_tiles, int n_tiles, int& t
 // every lane, and held in VGPRs across the main loop they cost registers the loop needs. The
 // grid is one-dimensional, the K slices included (slice-major, then tile_pos's order), so
 // the XCD order above gives each XCD a run of tiles of one K slice: its L2 then holds the few
-// A and B blocks of that K range which its workgroups share.
+// A and B blocks of that K range which its workgroups share. total: the workgroups, those of a
+// sliced tail not among them (then fewer than `tiles`: whole columns first).
 __device__ __forceinline__ void tile_of(int m_tiles, int tiles, int total, int64_t& tile_m,
                                         int64_t& tile_n, int& slice) {
   int t = tile_order(blockIdx.x, total);  // the grid is below 2^31 (host check)
   slice = __builtin_amdgcn_readfirstlane(t / tiles);
   int tm, tn;
-  tile_pos(t - slice * tiles, m_tiles, tiles / m_tiles, tm, tn);
+  tile_pos(t - slice * tiles, m_tiles, min(total, tiles) / m_tiles, tm, tn);
   tile_m = tm;
   tile_n = tn;
 }
@@ -1159,7 +1164,7 @@ __global__ __launch_bounds__(kThreads, STAGES == 2 ? 2 : 1) void hgemm_kernel(Ge
   const int tail_u = g.tail_splits > 0 ? (int)blockIdx.x - g.main_tiles : -1;
   if (tail_u >= 0) {
     int tm, tn;
-    tile_pos(g.main_tiles + tail_u / g.tail_splits, g.m_tiles, g.tiles / g.m_tiles, tm, tn);
+    tile_pos(g.main_tiles + tail_u / g.tail_splits, g.m_tiles, 0, tm, tn);
     const int64_t kt0 =
         (int64_t)__builtin_amdgcn_readfirstlane(tail_u % g.tail_splits) * g.kt_per_tail;
     hgemm_tile<NN, TA, EPI, true, BM, BM, STAGES>(g, tm, tn, kt0, kt0 + g.kt_per_tail, tail_u,
@@ -1422,7 +1427,7 @@ __global__ __launch_bounds__(kThreads, 1) void hgemm256_kernel(GemmArgs g) {
   const int tail_u = g.tail_splits > 0 ? (int)blockIdx.x - g.main_tiles : -1;
   if (tail_u >= 0) {
     int tm, tn;
-    tile_pos(g.main_tiles + tail_u / g.tail_splits, g.m_tiles, g.tiles / g.m_tiles, tm, tn);
+    tile_pos(g.main_tiles + tail_u / g.tail_splits, g.m_tiles, 0, tm, tn);
     const int kt0 = __builtin_amdgcn_readfirstlane(tail_u % g.tail_splits) * g.kt_per_tail;
     hgemm256_tile<NN, TA, EPI, true>(g, tm, tn, kt0, kt0 + g.kt_per_tail, tail_u, smem);
     return;
@@ -1444,9 +1449,7 @@ __global__ __launch_bounds__(256) void tail_reduce_kernel(GemmArgs g, int epi, i
   if (id >= (int64_t)tiles * per_tile) return;
   const int u = (int)(id / per_tile), w = (int)(id - (int64_t)u * per_tile);
   const int t = g.main_tiles + u;
-  int tm, tn;
-  tile_pos_lane(t, g.m_tiles, g.tiles / g.m_tiles, tm, tn);
-  const int64_t tile_m = tm, tile_n = tn;
+  const int64_t tile_m = t % g.m_tiles, tile_n = t / g.m_tiles;
   const int64_t slice = (int64_t)BM * BN;
   const float* part = g.tail_ws + (int64_t)u * g.tail_splits * slice;
   const int S = g.tail_splits;

@@ -228,6 +228,29 @@ def test_tile_major_order_equals_bnb_order(pkg, epi):
     assert torch.equal(torch.sort(scales).values, torch.sort(w.block_scales()).values)
 
 
+@pytest.mark.parametrize("M,N,K,tile,main", [(2048, 4608, 512, 128, 512), (3400, 4864, 512, 256, 256),
+                                             (1700, 9472, 256, 128, 1024)])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_sliced_tail_is_the_last_tiles_column_by_column(pkg, M, N, K, tile, main, mode):
+    """With more than 12 M tiles the tiles run in groups of M tiles, but the ones cut into K slices
+    are the last past the full rounds column by column (M fastest): the others keep the bits of the
+    product without slices, the sliced ones differ in summation order."""
+    L = pkg.linear
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    a = torch.randn(M, K, generator=g, device=DEV).half()
+    w = torch.randn(*((N, K) if mode == 0 else (K, N)), generator=g, device=DEV).half()
+    kw = dict(splits=1, tile=tile, stages=2)
+    sliced, whole = (L.hgemm(a, w, mode, tail=tail, **kw) for tail in (True, False))
+    rows = torch.arange(M, device=DEV)[:, None] // tile
+    cols = torch.arange(N, device=DEV)[None, :] // tile
+    tail = cols * (-(-M // tile)) + rows >= main
+    assert 0 < int(tail.sum()) < M * N
+    assert torch.equal(sliced[~tail], whole[~tail])
+    assert not torch.equal(sliced[tail], whole[tail])
+    want = a.double() @ (w.double().t() if mode == 0 else w.double())
+    assert rel_err(sliced, want) < 4e-4  # fp16 stores: 2^-12 at most, 2^-11 / sqrt(12) at random
+
+
 @pytest.mark.parametrize("mode,epi", [(0, 0), (0, 1), (0, 2), (0, 3), (1, 0), (1, 2)])
 def test_fp16_b_gemm_tail_slices(pkg, mode, epi):
     """One slice with a last round of at most 64 tiles: qlora_gemm16 given its workspace runs those
